@@ -457,7 +457,7 @@ size_t lagpm_estimate_box_bytes(const lagpm_params* p, size_t np) {
     const size_t real = f64 ? 8 : 4;
     const int L = lagpm_choose_cell_level(p->n, p->rsphere);
     const size_t mcell = (size_t)1 << L;
-    size_t b = np * (12 * 8 + 4 * 4 + 2 * 8 + 2 * 4);  // two sets of x..vz, id/id_alt/perm/perm2, keys, node counts
+    size_t b = (np + LAGPM_ARRAY_PAD) * 12 * 8 + np * (4 * 4 + 2 * 8 + 2 * 4);  // two sets of x..vz, id/id_alt/perm/perm2, keys, node counts
     b += np * (f64 ? 4 : 16);                             // pgroup / pp
     b += m * 8 + K * 2 * real + 4 * m * real;              // acc, padded FFT mesh, grad
     b += (f64 ? 4 : 8) * mcell * mcell * mcell + 4 * 8 + DSZ_COUNT * 4;  // cell roots, counters, sizes
@@ -489,10 +489,11 @@ int lagpm_box_create(lagpm_ctx* ctx, const lagpm_params* p, size_t np, lagpm_box
     do {                                                                \
         if (rc == LAGPM_OK) rc = dalloc(ctx, box, &(ptr), (cnt));       \
     } while (0)
-    ALLOC(box->x, np); ALLOC(box->y, np); ALLOC(box->z, np);
-    ALLOC(box->vx, np); ALLOC(box->vy, np); ALLOC(box->vz, np);
+    const size_t npad = np + LAGPM_ARRAY_PAD;
+    ALLOC(box->x, npad); ALLOC(box->y, npad); ALLOC(box->z, npad);
+    ALLOC(box->vx, npad); ALLOC(box->vy, npad); ALLOC(box->vz, npad);
     ALLOC(box->id, np); ALLOC(box->key, np); ALLOC(box->key2, np); ALLOC(box->perm, np); ALLOC(box->perm2, np);
-    for (int a = 0; a < 6; a++) ALLOC(box->alt[a], np);
+    for (int a = 0; a < 6; a++) ALLOC(box->alt[a], npad);
     ALLOC(box->id_alt, np); ALLOC(box->dfac, 4);
     ALLOC(box->acc, m);
     // one in-place FFT mesh (padded rows of 2(n/2+1)): density, then spectrum, then potential
@@ -571,6 +572,22 @@ int lagpm_box_set_cosmology(lagpm_box* box, double amax, double omep, double ome
 size_t lagpm_box_np(const lagpm_box* box) { return box ? box->np : 0; }
 size_t lagpm_box_device_bytes(const lagpm_box* box) { return box ? box->bytes : 0; }
 
+// waits for the queued upload; the box starts over as a new box would
+static int upload_done(lagpm_ctx* ctx, lagpm_box* box) {
+    HIPCHK(ctx, hipStreamSynchronize(box->st));
+    box->uploaded = true;
+    box->sorted = false;
+    box->tree_built = false;
+    // new particles: the box starts over as a new box would, with a full-depth first tree (the
+    // depth limit also sets how many key bits the sort orders, and so the particle order that
+    // the sums follow), so a box reused for other particles steps exactly as a fresh one
+    if (box->depth != LAGPM_KEY_BITS) {
+        box->depth = LAGPM_KEY_BITS;
+        lagpm_box_graphs_release(box);  // captured steps hold the old limit
+    }
+    return LAGPM_OK;
+}
+
 int lagpm_box_upload(lagpm_ctx* ctx, lagpm_box* box, const double* x, const double* y, const double* z, const double* vx,
                      const double* vy, const double* vz) {
     if (!ctx || !box || (box->np && (!x || !y || !z))) return lagpm_fail(ctx, LAGPM_E_INVAL, "NULL argument");
@@ -593,18 +610,7 @@ int lagpm_box_upload(lagpm_ctx* ctx, lagpm_box* box, const double* x, const doub
         hipLaunchKernelGGL(wrap_kernel, dim3(nblocks(np, 256)), dim3(256), 0, box->st, ps[a], np, (double)box->p.n);
     hipLaunchKernelGGL(iota_kernel, dim3(nblocks(np, 256)), dim3(256), 0, box->st, box->id, np);
     HIPCHK(ctx, hipGetLastError());
-    HIPCHK(ctx, hipStreamSynchronize(box->st));
-    box->uploaded = true;
-    box->sorted = false;
-    box->tree_built = false;
-    // new particles: the box starts over as a new box would, with a full-depth first tree (the
-    // depth limit also sets how many key bits the sort orders, and so the particle order that
-    // the sums follow), so a box reused for other particles steps exactly as a fresh one
-    if (box->depth != LAGPM_KEY_BITS) {
-        box->depth = LAGPM_KEY_BITS;
-        lagpm_box_graphs_release(box);  // captured steps hold the old limit
-    }
-    return LAGPM_OK;
+    return upload_done(ctx, box);
 }
 
 int lagpm_box_download(lagpm_ctx* ctx, lagpm_box* box, double* x, double* y, double* z, double* vx, double* vy, double* vz) {
@@ -626,11 +632,12 @@ int lagpm_box_upload_eunha(lagpm_ctx* ctx, lagpm_box* box, const void* dm_bp, si
     if (!ctx || !box || (np && !dm_bp)) return lagpm_fail(ctx, LAGPM_E_INVAL, "NULL argument");
     if (np != box->np) return lagpm_fail(ctx, LAGPM_E_INVAL, "particle count differs from the box");
     if (nx != box->p.n) return lagpm_fail(ctx, LAGPM_E_INVAL, "nx differs from the box mesh size");
-    std::vector<double> a(6 * np);
-    double* q = a.data();
-    if (lagpm_eunha_decode(dm_bp, np, nx, q, q + np, q + 2 * np, q + 3 * np, q + 4 * np, q + 5 * np) != LAGPM_OK)
-        return lagpm_fail(ctx, LAGPM_E_INVAL, "bad particle records");
-    return lagpm_box_upload(ctx, box, q, q + np, q + 2 * np, q + 3 * np, q + 4 * np, q + 5 * np);
+    if (np == 0) {
+        box->uploaded = true;
+        return LAGPM_OK;
+    }
+    RCHK(lagpm_upload_records(ctx, box, dm_bp));
+    return upload_done(ctx, box);
 }
 
 int lagpm_box_download_eunha_vel(lagpm_ctx* ctx, lagpm_box* box, void* dm_bp, size_t np) {

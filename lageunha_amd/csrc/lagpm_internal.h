@@ -17,6 +17,10 @@
 #define LAGPM_MAX_INDEX (1u << 27)  // particles per box: walk lists pack (index << 5 | neighbour) in 32 bits
 #define LAGPM_MAX_NODES (1u << 26)  // nodes per box: walk stacks pack (node << 5 | neighbour) in a non-negative int
 
+// Entries past the last particle of the box's FP64 particle arrays and their scratch twins, so that
+// four scratch arrays hold the particles as 32-byte records, a quarter (rounded up) each.
+#define LAGPM_ARRAY_PAD 4
+
 // Doubles in the static power-spectrum scratch of each device: pk and npk bins for n <= 4096.
 #define LAGPM_PK_SCRATCH_DOUBLES (2 * (4096 + 1))
 
@@ -239,6 +243,10 @@ int lagpm_exclusive_scan_u32(lagpm_ctx* ctx, hipStream_t s, uint32_t* tmp, const
 int lagpm_radix_sort_pairs(lagpm_ctx* ctx, hipStream_t s, uint32_t* tmp, uint64_t* key, uint64_t* key_alt, uint32_t* val,
                            uint32_t* val_alt, size_t n, int bits, bool* result_in_alt,
                            int lo_bit = 0);
+
+// ---- records (records.hip) ----
+// Copies np 32-byte GOTPM records to the device and decodes them into the box's particle arrays.
+int lagpm_upload_records(lagpm_ctx* ctx, lagpm_box* box, const void* dm_bp);
 
 // ---- PM (pm.hip) ----
 int lagpm_pm_deposit(lagpm_ctx* ctx, lagpm_box* box);          // fills acc and rho

@@ -1,0 +1,87 @@
+// records.hip — GOTPM particle records on the device: decoding on upload (XofP/YofP/ZofP,
+// eunha.h:1212, 1228-1232).
+//
+// A record is 32 bytes (dmparticletype under GOTPM + XYZDBL, eunha.h:389-399): u64 index|flag, f32
+// displacement from the lattice site, f32 velocity. The host moves whole records and the device
+// turns them into the box's FP64 arrays: one pass over HBM, where the same loop on one host thread
+// (three fmod and three 64-bit divisions a record) took most of an upload.
+#include "lagpm_internal.h"
+
+namespace {
+
+// one record as two 16-byte words
+struct rec32 {
+    ulonglong2 a;  // index|flag, (x, y)
+    ulonglong2 b;  // (z, vx), (vy, vz)
+};
+static_assert(sizeof(rec32) == 32, "GOTPM particle is 32 bytes");
+
+__device__ inline float lo_f(unsigned long long w) { return __uint_as_float((uint32_t)w); }
+__device__ inline float hi_f(unsigned long long w) { return __uint_as_float((uint32_t)(w >> 32)); }
+
+// lattice site of the low 56 bits of the index word: idx = i + n (j + n k)
+__device__ inline void lattice_site(unsigned long long u4if, uint32_t n, double s[3]) {
+    const unsigned long long idx = (u4if << 8) >> 8;  // PINDX, eunha.h:1212
+    if (idx <= 0xffffffffull) {  // 32-bit divisions (64-bit ones are a software loop)
+        const uint32_t q = (uint32_t)idx, r = q / n;
+        s[0] = (double)(q - r * n);
+        s[1] = (double)(r % n);
+        s[2] = (double)(r / n);
+    } else {
+        const unsigned long long r = idx / n;
+        s[0] = (double)(idx - r * n);
+        s[1] = (double)(r % n);
+        s[2] = (double)(r / n);
+    }
+}
+
+// XofP = fmod(dx + i + nx, nx), then wrapped into [0, nx) as every upload is (a displacement below
+// -nx leaves a negative remainder)
+__device__ inline double decode_pos(float d, double site, double L) {
+    double v = fmod((double)d + site + L, L);
+    if (v < 0) v += L;
+    if (v >= L) v = 0.0;
+    return v;
+}
+
+// Bound by HBM: 32 bytes read and 52 written a record (the copy over PCIe takes longer). An upload of
+// 2.1M records: 90 ms with the host loop and the copies of its 48 bytes a record, 5 ms with this.
+__global__ void __launch_bounds__(256) decode_records_kernel(const rec32* __restrict__ rec, size_t first, size_t count, uint32_t n,
+                                                             double* __restrict__ x, double* __restrict__ y, double* __restrict__ z,
+                                                             double* __restrict__ vx, double* __restrict__ vy,
+                                                             double* __restrict__ vz, uint32_t* __restrict__ id) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= count) return;
+    const ulonglong2 a = rec[t].a, b = rec[t].b;
+    double s[3];
+    lattice_site(a.x, n, s);
+    const double L = (double)n;
+    const size_t i = first + t;
+    x[i] = decode_pos(lo_f(a.y), s[0], L);
+    y[i] = decode_pos(hi_f(a.y), s[1], L);
+    z[i] = decode_pos(lo_f(b.x), s[2], L);
+    vx[i] = (double)hi_f(b.x);
+    vy[i] = (double)lo_f(b.y);
+    vz[i] = (double)hi_f(b.y);
+    id[i] = (uint32_t)i;
+}
+
+unsigned grid_of(size_t n) { return (unsigned)((n + 255) / 256); }
+
+}  // namespace
+
+// The records pass through four of the box's scratch arrays (alt, free between sorts), a quarter of
+// them each: their 8 bytes a particle hold the quarter's 32 bytes a record.
+int lagpm_upload_records(lagpm_ctx* ctx, lagpm_box* box, const void* dm_bp) {
+    const size_t np = box->np, q = (np + 3) / 4;
+    static_assert(LAGPM_ARRAY_PAD * 8 >= 32, "a quarter rounded up fits its scratch array");
+    for (size_t k = 0, first = 0; first < np; k++, first += q) {
+        const size_t cnt = std::min(q, np - first);
+        HIPCHK(ctx, hipMemcpyAsync(box->alt[k], (const char*)dm_bp + first * sizeof(rec32), cnt * sizeof(rec32),
+                                   hipMemcpyHostToDevice, box->st));
+        hipLaunchKernelGGL(decode_records_kernel, dim3(grid_of(cnt)), dim3(256), 0, box->st, (const rec32*)box->alt[k], first, cnt,
+                           (uint32_t)box->p.n, box->x, box->y, box->z, box->vx, box->vy, box->vz, box->id);
+        HIPCHK(ctx, hipGetLastError());
+    }
+    return LAGPM_OK;
+}
