@@ -643,18 +643,13 @@ int lagpm_box_upload_eunha(lagpm_ctx* ctx, lagpm_box* box, const void* dm_bp, si
 int lagpm_box_download_eunha_vel(lagpm_ctx* ctx, lagpm_box* box, void* dm_bp, size_t np) {
     if (!ctx || !box || (np && !dm_bp)) return lagpm_fail(ctx, LAGPM_E_INVAL, "NULL argument");
     if (np != box->np) return lagpm_fail(ctx, LAGPM_E_INVAL, "particle count differs from the box");
-    std::vector<double> v(3 * np);
-    RCHK(lagpm_box_download(ctx, box, nullptr, nullptr, nullptr, v.data(), v.data() + np, v.data() + 2 * np));
-    return lagpm_eunha_encode(dm_bp, np, box->p.n, nullptr, nullptr, nullptr, v.data(), v.data() + np, v.data() + 2 * np);
+    return np ? lagpm_download_records(ctx, box, dm_bp, false) : LAGPM_OK;
 }
 
 int lagpm_box_download_eunha(lagpm_ctx* ctx, lagpm_box* box, void* dm_bp, size_t np) {
     if (!ctx || !box || (np && !dm_bp)) return lagpm_fail(ctx, LAGPM_E_INVAL, "NULL argument");
     if (np != box->np) return lagpm_fail(ctx, LAGPM_E_INVAL, "particle count differs from the box");
-    std::vector<double> a(6 * np);
-    double* q = a.data();
-    RCHK(lagpm_box_download(ctx, box, q, q + np, q + 2 * np, q + 3 * np, q + 4 * np, q + 5 * np));
-    return lagpm_eunha_encode(dm_bp, np, box->p.n, q, q + np, q + 2 * np, q + 3 * np, q + 4 * np, q + 5 * np);
+    return np ? lagpm_download_records(ctx, box, dm_bp, true) : LAGPM_OK;
 }
 
 static int pm_factor(lagpm_ctx* ctx, const lagpm_evolfact* ef, int pmstatus, double* f) {

@@ -247,6 +247,8 @@ int lagpm_radix_sort_pairs(lagpm_ctx* ctx, hipStream_t s, uint32_t* tmp, uint64_
 // ---- records (records.hip) ----
 // Copies np 32-byte GOTPM records to the device and decodes them into the box's particle arrays.
 int lagpm_upload_records(lagpm_ctx* ctx, lagpm_box* box, const void* dm_bp);
+// Writes the particles' velocities (and displacements) into np records in the caller's memory.
+int lagpm_download_records(lagpm_ctx* ctx, lagpm_box* box, void* dm_bp, bool positions);
 
 // ---- PM (pm.hip) ----
 int lagpm_pm_deposit(lagpm_ctx* ctx, lagpm_box* box);          // fills acc and rho

@@ -1,5 +1,5 @@
 // records.hip — GOTPM particle records on the device: decoding on upload (XofP/YofP/ZofP,
-// eunha.h:1212, 1228-1232).
+// eunha.h:1212, 1228-1232) and its inverse on download.
 //
 // A record is 32 bytes (dmparticletype under GOTPM + XYZDBL, eunha.h:389-399): u64 index|flag, f32
 // displacement from the lattice site, f32 velocity. The host moves whole records and the device
@@ -45,7 +45,7 @@ __device__ inline double decode_pos(float d, double site, double L) {
 }
 
 // Bound by HBM: 32 bytes read and 52 written a record (the copy over PCIe takes longer). An upload of
-// 2.1M records: 90 ms with the host loop and the copies of its 48 bytes a record, 5 ms with this.
+// 2.1M records: 90 ms with the host loop and the copies of its 48 bytes a record, 2.4 ms with this.
 __global__ void __launch_bounds__(256) decode_records_kernel(const rec32* __restrict__ rec, size_t first, size_t count, uint32_t n,
                                                              double* __restrict__ x, double* __restrict__ y, double* __restrict__ z,
                                                              double* __restrict__ vx, double* __restrict__ vy,
@@ -66,6 +66,47 @@ __global__ void __launch_bounds__(256) decode_records_kernel(const rec32* __rest
     id[i] = (uint32_t)i;
 }
 
+// the displacement from the record's own lattice site, taken as the periodic image nearest to it
+// ([-n/2, n/2)), so XofP of the record gives the position back
+__device__ inline uint32_t encode_pos(double pos, double site, double L) {
+    const double h = 0.5 * L;
+    double d = fmod(pos - site, L);
+    if (d >= h) d -= L;
+    if (d < -h) d += L;
+    return __float_as_uint((float)d);
+}
+
+struct rec_quarters {
+    uint32_t* p[4];  // records of 8 words, `q` of them in each
+    uint32_t q;
+};
+// Particle i of the box's order is record id[i]: its index word is read there and the fields beside
+// it are written (POS: displacement and velocity, otherwise the velocity alone). A record is half a
+// 64-byte sector, so a particle touches one sector of the records however they are ordered.
+template <bool POS>
+__global__ void __launch_bounds__(256) encode_records_kernel(rec_quarters Q, size_t np, uint32_t n, const double* __restrict__ x,
+                                                             const double* __restrict__ y, const double* __restrict__ z,
+                                                             const double* __restrict__ vx, const double* __restrict__ vy,
+                                                             const double* __restrict__ vz, const uint32_t* __restrict__ id) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    const uint32_t r = id[i], k = r / Q.q;
+    uint32_t* rec = Q.p[k] + 8 * (size_t)(r - k * Q.q);
+    const uint32_t ux = __float_as_uint((float)vx[i]), uy = __float_as_uint((float)vy[i]), uz = __float_as_uint((float)vz[i]);
+    if constexpr (POS) {
+        const unsigned long long u4if = *reinterpret_cast<const unsigned long long*>(rec);
+        double s[3];
+        lattice_site(u4if, n, s);
+        const double L = (double)n;
+        rec[2] = encode_pos(x[i], s[0], L);
+        rec[3] = encode_pos(y[i], s[1], L);
+        rec[4] = encode_pos(z[i], s[2], L);
+    }
+    rec[5] = ux;
+    rec[6] = uy;
+    rec[7] = uz;
+}
+
 unsigned grid_of(size_t n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
@@ -83,5 +124,25 @@ int lagpm_upload_records(lagpm_ctx* ctx, lagpm_box* box, const void* dm_bp) {
                            (uint32_t)box->p.n, box->x, box->y, box->z, box->vx, box->vy, box->vz, box->id);
         HIPCHK(ctx, hipGetLastError());
     }
+    return LAGPM_OK;
+}
+
+// The caller's records (their index words name the lattice sites) go to the device, get their fields
+// there and come back whole: two copies at PCIe rate, where copying six FP64 arrays back and filling
+// the records on one host thread took 39 ms for 2.1M records (this: 6.4 ms).
+int lagpm_download_records(lagpm_ctx* ctx, lagpm_box* box, void* dm_bp, bool positions) {
+    const size_t np = box->np, q = (np + 3) / 4;
+    rec_quarters Q;
+    Q.q = (uint32_t)q;
+    for (int k = 0; k < 4; k++) Q.p[k] = reinterpret_cast<uint32_t*>(box->alt[k]);
+    for (size_t k = 0, first = 0; first < np; k++, first += q)
+        HIPCHK(ctx, hipMemcpyAsync(box->alt[k], (const char*)dm_bp + first * sizeof(rec32), std::min(q, np - first) * sizeof(rec32),
+                                   hipMemcpyHostToDevice, box->st));
+    auto kern = positions ? encode_records_kernel<true> : encode_records_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3(grid_of(np)), dim3(256), 0, box->st, Q, np, (uint32_t)box->p.n, box->x, box->y, box->z, box->vx,
+                       box->vy, box->vz, box->id);
+    HIPCHK(ctx, hipGetLastError());
+    for (size_t k = 0, first = 0; first < np; k++, first += q)
+        RCHK(lagpm_d2h(ctx, (char*)dm_bp + first * sizeof(rec32), box->alt[k], std::min(q, np - first) * sizeof(rec32), box->st));
     return LAGPM_OK;
 }

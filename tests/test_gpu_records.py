@@ -38,3 +38,29 @@ def test_upload_decodes_as_the_host_does(ctx, count, precision):
         b.upload_eunha(rec)
         got, gv = b.download()
     assert np.array_equal(got, pos) and np.array_equal(gv, vel)
+
+
+@pytest.mark.parametrize("count", [1, 2, 3, 5, 255, 257, 70001])
+@pytest.mark.parametrize("precision", [lagpm.PREC_FP32, lagpm.PREC_FP64])
+def test_download_encodes_as_the_host_does(ctx, count, precision):
+    """After a sort (the box's order is not the caller's), into records with other sites than the
+    uploaded ones; every byte of the records, kept fields included."""
+    n = 24
+    rec = make_records(n, count, count + 1)
+    into = make_records(n, count, count + 2)
+    into["x"][::3] = np.float32(np.nan)  # overwritten by a full download, kept by a velocity one
+    with lagpm.Box(ctx, lagpm.make_params(n, precision=precision), count) as b:
+        b.upload_eunha(rec)
+        b.pmmain(lagpm.evolfact(1.0), lagpm.KICK)
+        b.drift(0.7)
+        pos, vel = b.download()
+        for full in (True, False):
+            want, got = into.copy(), into.copy()
+            if full:
+                lagpm.eunha_encode(want, n, pos, vel)
+                b.download_eunha(got)
+            else:
+                for c, a in enumerate("xyz"):
+                    want["v" + a] = vel[:, c].astype(np.float32)
+                b.download_eunha_vel(got)
+            assert got.tobytes() == want.tobytes()
