@@ -673,31 +673,11 @@ static int need_particles(lagpm_ctx* ctx, lagpm_box* box) {
     return LAGPM_OK;
 }
 
-// n^3 host values <-> the padded FFT mesh (rows of n values every 2(n/2+1))
-static int mesh_copy(lagpm_ctx* ctx, lagpm_box* box, void* host, bool to_host, size_t elem) {
-    const size_t n = (size_t)box->p.n, mx = 2 * (n / 2 + 1);
-    if (to_host)
-        HIPCHK(ctx, hipMemcpy2DAsync(host, n * elem, box->rho, mx * elem, n * elem, n * n, hipMemcpyDeviceToHost, box->st));
-    else
-        HIPCHK(ctx, hipMemcpy2DAsync(box->rho, mx * elem, host, n * elem, n * elem, n * n, hipMemcpyHostToDevice, box->st));
-    return LAGPM_OK;
-}
-
 int lagpm_tsc(lagpm_ctx* ctx, lagpm_box* box, float* den) {
     RCHK(need_particles(ctx, box));
     if (!box->sorted) RCHK(lagpm_sort_particles(ctx, box));
     RCHK(lagpm_pm_deposit(ctx, box));
-    if (den) {
-        const size_t m = (size_t)box->p.n * box->p.n * box->p.n;
-        if (box->p.precision == LAGPM_PREC_FP64) {
-            std::vector<double> t(m);
-            RCHK(mesh_copy(ctx, box, t.data(), true, 8));
-            HIPCHK(ctx, hipStreamSynchronize(box->st));
-            for (size_t i = 0; i < m; i++) den[i] = (float)t[i];
-        } else {
-            RCHK(mesh_copy(ctx, box, den, true, 4));
-        }
-    }
+    if (den) return lagpm_mesh_download(ctx, box, den);
     HIPCHK(ctx, hipStreamSynchronize(box->st));
     return LAGPM_OK;
 }
@@ -716,17 +696,7 @@ int lagpm_tsc_fixed(lagpm_ctx* ctx, lagpm_box* box, int64_t* acc, int* scale_bit
 int lagpm_psolver(lagpm_ctx* ctx, lagpm_box* box, float* phi) {
     RCHK(need_particles(ctx, box));
     RCHK(lagpm_pm_solve(ctx, box));
-    if (phi) {
-        const size_t m = (size_t)box->p.n * box->p.n * box->p.n;
-        if (box->p.precision == LAGPM_PREC_FP64) {
-            std::vector<double> t(m);
-            RCHK(mesh_copy(ctx, box, t.data(), true, 8));
-            HIPCHK(ctx, hipStreamSynchronize(box->st));
-            for (size_t i = 0; i < m; i++) phi[i] = (float)t[i];
-        } else {
-            RCHK(mesh_copy(ctx, box, phi, true, 4));
-        }
-    }
+    if (phi) return lagpm_mesh_download(ctx, box, phi);
     HIPCHK(ctx, hipStreamSynchronize(box->st));
     return LAGPM_OK;
 }
@@ -761,16 +731,7 @@ int lagpm_fda4(lagpm_ctx* ctx, lagpm_box* box, const lagpm_evolfact* ef, int pms
 
 int lagpm_set_potential(lagpm_ctx* ctx, lagpm_box* box, const float* phi) {
     if (!ctx || !box || !phi) return lagpm_fail(ctx, LAGPM_E_INVAL, "NULL argument");
-    const size_t m = (size_t)box->p.n * box->p.n * box->p.n;
-    if (box->p.precision == LAGPM_PREC_FP64) {
-        std::vector<double> t(phi, phi + m);
-        RCHK(mesh_copy(ctx, box, t.data(), false, 8));
-        HIPCHK(ctx, hipStreamSynchronize(box->st));
-    } else {
-        RCHK(mesh_copy(ctx, box, (void*)phi, false, 4));
-        HIPCHK(ctx, hipStreamSynchronize(box->st));
-    }
-    return LAGPM_OK;
+    return lagpm_mesh_upload(ctx, box, phi);
 }
 
 int lagpm_get_gradient(lagpm_ctx* ctx, lagpm_box* box, float* grad4) {

@@ -260,6 +260,9 @@ int lagpm_green_device(lagpm_ctx* ctx, hipStream_t s, int n, int prec, double ef
 int lagpm_green_prepare(lagpm_ctx* ctx, hipStream_t s, int n, double efold, int deconvolve);
 size_t lagpm_deposit_chunk_cap(int n, size_t np);
 size_t lagpm_deposit_blocks(int n);  // Morton blocks of the deposit's chunking
+// the resident padded mesh (density or potential) to and from n^3 floats of the caller; waits
+int lagpm_mesh_download(lagpm_ctx* ctx, lagpm_box* box, float* host);
+int lagpm_mesh_upload(lagpm_ctx* ctx, lagpm_box* box, const float* host);
 int lagpm_fft_release(lagpm_ctx* ctx);
 int lagpm_box_fft_release(lagpm_box* box);
 int lagpm_pm_prepare(lagpm_ctx* ctx, lagpm_box* box);
