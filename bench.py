@@ -289,13 +289,11 @@ def ensemble(args, ctx, lagpm, ics):
         lat["batched"].append(time.perf_counter() - t)
     tt["batched"] = time.perf_counter() - t0
     log(f"[bench] ensemble batched: {tt['batched']:.2f} s")
-    # the same batched steps with every kernel launched (no step graphs), for comparison
-    ctx.set_step_graphs(False)
+    # two more batched steps: every kernel is launched in these as in the ones above (no step graphs)
     t0 = time.perf_counter()
     for s in range(2):
         lagpm.batch_step(ctx, sets["batched"], a0 + da * (steps + 1 + s), da)
     t_eager = (time.perf_counter() - t0) / 2
-    ctx.set_step_graphs(True)
     for s in range(2):  # keep the plain set in step with the batched one
         for bx in sets["plain"]:
             bx.kdk_step(a0 + da * (steps + 1 + s), da)
@@ -488,7 +486,7 @@ def main():
 
     def step():
         # one GOTPM step through the whole-step entry point: drag, sort and tree build, then the
-        # walk beside the PM kick, then drift (step graphs on)
+        # walk beside the PM kick, then drift
         box.kdk_step(1.0, 0.25)
 
     # first step traced phase by phase (synchronised), so a slow phase names itself
@@ -513,8 +511,8 @@ def main():
         t0 = time.perf_counter()
         for i in range(args.steps):
             step()
-            # the walk runs outside the step graphs, between HIP events on the context stream (the
-            # stream it is launched on); the step has completed when kdk_step returns
+            # the walk runs between HIP events on the context stream (the stream it is launched on);
+            # the step has completed when kdk_step returns
             walk_ms.append(box.timings().ms_walk)
             s = box.tree_stats()
             walk_stats.append((s.n_pp, s.n_pc))
@@ -522,15 +520,14 @@ def main():
         t1 = time.perf_counter()
     ms = (t1 - t0) * 1e3 / args.steps
     log(f"[bench] timed {args.steps} steps: {ms:.2f} ms/step")
-    # per-phase device times: two more steps with the kernels launched eagerly (phase events are
-    # not recorded inside graphs); the PM phases overlap the walk there as in the timed steps
+    # per-phase device times: two more steps with the phase events (which turning step graphs off
+    # by a call records); the PM phases overlap the tree build there as in the timed steps
     ctx.set_step_graphs(False)
     for i in range(2):
         step()
         phases.append(box.timings().as_dict())
         s = box.tree_stats()
         stats.append((s.n_pp, s.n_pc, s.n_nodes, s.n_groups))
-    ctx.set_step_graphs(True)
     # one more step with the walk counting the evaluated pairs within the cutoff (slower, untimed)
     ctx.set_walk_census(True)
     step()

@@ -1161,15 +1161,19 @@ void front_host_effects(lagpm_box* b) {
 }
 
 // Everything of one box's step before the walk, queued on box->st (and box->st2), then the event
-// the walk waits for (ev[13]). With graphs on, the front is captured once per particle-set parity
-// and replayed; factors are written first.
+// the walk waits for (ev[13]). With step graphs turned on, the front is captured once per
+// particle-set parity and replayed; factors are written first.
 int step_front(lagpm_ctx* ctx, lagpm_box* box, const lagpm_evolfact& ef) {
     hipLaunchKernelGGL(set_factors_kernel, dim3(1), dim3(64), 0, box->st, box->dfac, (double)ef.fact1, (double)ef.fact2,
                        (double)ef.pfact, 7);
     HIPCHK(ctx, hipGetLastError());
     auto eager = [&]() -> int {
-        RCHK(front_body(ctx, box, box->ev));
-        box->pm_timed = true;
+        if (!ctx->step_events) {  // the events that every step's tree times need
+            HIPCHK(ctx, hipEventRecord(box->ev[8], box->st));
+            HIPCHK(ctx, hipEventRecord(box->ev[9], box->st));
+        }
+        RCHK(front_body(ctx, box, ctx->step_events ? box->ev : nullptr));
+        box->pm_timed = ctx->step_events;
         HIPCHK(ctx, hipEventRecord(box->ev[13], box->st));
         return LAGPM_OK;
     };
@@ -1429,6 +1433,7 @@ int lagpm_batch_step(lagpm_ctx* ctx, lagpm_box* const* boxes, int nbox, const do
 int lagpm_set_step_graphs(lagpm_ctx* ctx, int enable) {
     if (!ctx) return LAGPM_E_INVAL;
     ctx->use_graphs = enable != 0;
+    ctx->step_events = enable == 0;
     return LAGPM_OK;
 }
 

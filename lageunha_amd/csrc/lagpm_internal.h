@@ -69,7 +69,8 @@ struct lagpm_ctx {
     walk_box* walk_boxes = nullptr;          // descriptor array of the last launch
     uint32_t* walk_prefix = nullptr;         // group prefix over the descriptors
     size_t walk_box_cap = 0;
-    bool use_graphs = true;                  // capture box step fronts in hipGraphs
+    bool use_graphs = false;                 // capture box step fronts in hipGraphs (lagpm_set_step_graphs)
+    bool step_events = false;                // record the phase events of step fronts (lagpm_set_step_graphs(ctx, 0))
     bool walk_census = false;                // FP32 walks count the pairs within the cutoff
     int batch_stages = 5;                    // groups of a pipelined batch step (1: no pipeline)
     int stage_reserve_cu = 32;               // CUs a non-final group's walk leaves to the next fronts
