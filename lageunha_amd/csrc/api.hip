@@ -84,12 +84,13 @@ __global__ void drift_kernel(double* __restrict__ x, double* __restrict__ y, dou
     z[i] = p[2];
 }
 
-// v += tv: a tree kick computed on its own (see the walk) applied to the velocities
+// v += tv: a tree kick computed on its own (see the walk) applied to the velocities. A build that
+// overflowed its node arrays was not walked, so tv holds no kick (the call redoes the tree).
 __global__ void add3_kernel(double* __restrict__ vx, double* __restrict__ vy, double* __restrict__ vz,
                             const double* __restrict__ tvx, const double* __restrict__ tvy, const double* __restrict__ tvz,
-                            size_t np) {
+                            size_t np, const uint32_t* __restrict__ dsz) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= np) return;
+    if (i >= np || dsz[DSZ_OVERFLOW]) return;
     vx[i] += tvx[i];
     vy[i] += tvy[i];
     vz[i] += tvz[i];
@@ -845,7 +846,8 @@ static int tree_enqueue(lagpm_ctx* ctx, lagpm_box* box, double fact, bool combin
         if (box->st != ctx->stream) HIPCHK(ctx, hipStreamWaitEvent(box->st, ev[3], 0));
         if (combine) {
             hipLaunchKernelGGL(add3_kernel, dim3(nblocks(box->np, 256)), dim3(256), 0, box->st, box->vx, box->vy, box->vz,
-                               (const double*)box->alt[0], (const double*)box->alt[1], (const double*)box->alt[2], box->np);
+                               (const double*)box->alt[0], (const double*)box->alt[1], (const double*)box->alt[2], box->np,
+                               (const uint32_t*)box->dsz);
             HIPCHK(ctx, hipGetLastError());
         }
     }
