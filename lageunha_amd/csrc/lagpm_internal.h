@@ -53,6 +53,7 @@ struct walk_box;  // device view of one box for the walk (tree.hip)
 
 // XCDs of one MI355X in SPX mode: the walk splits its groups into this many ranges.
 constexpr int LAGPM_WALK_XCDS = 8;
+constexpr int LAGPM_TICKET_STRIDE = 32;  // words from one range's ticket counter to the next: a 128-byte line each
 
 struct lagpm_ctx {
     int device = 0;
@@ -65,7 +66,7 @@ struct lagpm_ctx {
     // walk resources (every walk runs on `stream`, so one set serves all boxes)
     int* walk_stack = nullptr;
     size_t walk_stack_entries = 0;
-    unsigned long long* walk_ticket = nullptr;  // LAGPM_WALK_XCDS group tickets, one per XCD range
+    uint32_t* walk_ticket = nullptr;  // group tickets, one per XCD range, a line each
     walk_box* walk_boxes = nullptr;          // descriptor array of the last launch
     uint32_t* walk_prefix = nullptr;         // group prefix over the descriptors
     size_t walk_box_cap = 0;
