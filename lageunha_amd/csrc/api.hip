@@ -366,14 +366,6 @@ int lagpm_get_tables(lagpm_ctx* ctx, const lagpm_params* p, const law_tables** o
     return LAGPM_OK;
 }
 
-int lagpm_d2h(lagpm_ctx* ctx, void* dst, const void* src, size_t bytes, hipStream_t s) {
-    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-    const hipError_t w = hipStreamSynchronize(s);
-    if (e != hipSuccess) return lagpm_fail(ctx, LAGPM_E_HIP, std::string("device-to-host copy: ") + hipGetErrorString(e));
-    if (w != hipSuccess) return lagpm_fail(ctx, LAGPM_E_HIP, std::string("device-to-host copy (wait): ") + hipGetErrorString(w));
-    return LAGPM_OK;
-}
-
 extern "C" {
 
 int lagpm_abi_version(void) { return LAGPM_ABI_VERSION; }
@@ -433,6 +425,7 @@ int lagpm_destroy(lagpm_ctx* ctx) {
     dfree(ctx->walk_ticket);
     dfree(ctx->walk_boxes);
     dfree(ctx->walk_prefix);
+    lagpm_stager_release(ctx);
     if (ctx->readback) (void)hipHostFree(ctx->readback);
     if (ctx->readback1) (void)hipHostFree(ctx->readback1);
     for (int i = 0; i < 4; i++)
@@ -597,15 +590,15 @@ int lagpm_box_upload(lagpm_ctx* ctx, lagpm_box* box, const double* x, const doub
         box->uploaded = true;
         return LAGPM_OK;
     }
-    HIPCHK(ctx, hipMemcpyAsync(box->x, x, b, hipMemcpyHostToDevice, box->st));
-    HIPCHK(ctx, hipMemcpyAsync(box->y, y, b, hipMemcpyHostToDevice, box->st));
-    HIPCHK(ctx, hipMemcpyAsync(box->z, z, b, hipMemcpyHostToDevice, box->st));
-    double* vs[3] = {box->vx, box->vy, box->vz};
-    const double* hs[3] = {vx, vy, vz};
-    for (int a = 0; a < 3; a++) {
-        if (hs[a]) HIPCHK(ctx, hipMemcpyAsync(vs[a], hs[a], b, hipMemcpyHostToDevice, box->st));
-        else HIPCHK(ctx, hipMemsetAsync(vs[a], 0, b, box->st));
+    double* to[6] = {box->x, box->y, box->z, box->vx, box->vy, box->vz};
+    const double* from[6] = {x, y, z, vx, vy, vz};
+    lagpm_segment seg[6];
+    size_t nseg = 0;
+    for (int a = 0; a < 6; a++) {
+        if (from[a]) seg[nseg++] = {to[a], const_cast<double*>(from[a]), b};
+        else HIPCHK(ctx, hipMemsetAsync(to[a], 0, b, box->st));
     }
+    RCHK(lagpm_copy_segments(ctx, seg, nseg, false, box->st));
     double* ps[3] = {box->x, box->y, box->z};
     for (int a = 0; a < 3; a++)
         hipLaunchKernelGGL(wrap_kernel, dim3(nblocks(np, 256)), dim3(256), 0, box->st, ps[a], np, (double)box->p.n);
@@ -619,13 +612,15 @@ int lagpm_box_download(lagpm_ctx* ctx, lagpm_box* box, double* x, double* y, dou
     const size_t np = box->np;
     double* src[6] = {box->x, box->y, box->z, box->vx, box->vy, box->vz};
     double* dst[6] = {x, y, z, vx, vy, vz};
+    lagpm_segment seg[6];
+    size_t nseg = 0;
     for (int a = 0; a < 6; a++) {
         if (!dst[a] || np == 0) continue;
-        hipLaunchKernelGGL(scatter_kernel, dim3(nblocks(np, 256)), dim3(256), 0, box->st, src[a], box->id, np, box->alt[0]);
+        hipLaunchKernelGGL(scatter_kernel, dim3(nblocks(np, 256)), dim3(256), 0, box->st, src[a], box->id, np, box->alt[a]);
         HIPCHK(ctx, hipGetLastError());
-        RCHK(lagpm_d2h(ctx, dst[a], box->alt[0], np * sizeof(double), box->st));
+        seg[nseg++] = {box->alt[a], dst[a], np * sizeof(double)};
     }
-    return LAGPM_OK;
+    return nseg ? lagpm_copy_segments(ctx, seg, nseg, true, box->st) : LAGPM_OK;
 }
 
 // GOTPM + XYZDBL particle: u64 index|flag (flag in the top byte), f32 dx,dy,dz, f32 vx,vy,vz.

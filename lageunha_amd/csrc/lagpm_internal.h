@@ -49,6 +49,8 @@ struct law_tables {
     double* tabd = nullptr;   // 6 per bin: d0 s0 d1 s1 d2 s2 (FP64 walk)
 };
 
+struct lagpm_stager;  // pinned slots of host copies (transfer.hip)
+
 struct walk_box;  // device view of one box for the walk (tree.hip)
 
 // XCDs of one MI355X in SPX mode: the walk splits its groups into this many ranges.
@@ -84,6 +86,7 @@ struct lagpm_ctx {
     void* readback = nullptr;
     size_t readback_count = 0;
     void* readback1 = nullptr;
+    lagpm_stager* stager = nullptr;  // made by the first large host copy
 };
 
 // Tunables of the tree correction (chosen per box; the autotuner may override).
@@ -233,6 +236,15 @@ int lagpm_fail(lagpm_ctx* ctx, int code, const std::string& msg);
 // the outcome: the stream is synchronised even when queuing the copy fails, so no copy can still
 // be writing into host memory the caller is about to free or leave (stack buffers included).
 int lagpm_d2h(lagpm_ctx* ctx, void* dst, const void* src, size_t bytes, hipStream_t s);
+// Host-to-device copy queued on stream s; the host memory is the caller's again when it returns.
+int lagpm_h2d(lagpm_ctx* ctx, void* dst, const void* src, size_t bytes, hipStream_t s);
+// Several such copies in one go (transfer.hip).
+struct lagpm_segment {
+    void *dev, *host;
+    size_t bytes;
+};
+int lagpm_copy_segments(lagpm_ctx* ctx, const lagpm_segment* seg, size_t nseg, bool to_host, hipStream_t s);
+void lagpm_stager_release(lagpm_ctx* ctx);
 
 // ---- scans / sort (sort.hip) ----
 // Scratch bytes a box needs for scans of n entries and for a radix sort of n keys.
