@@ -322,8 +322,8 @@ int lagpm_drift(lagpm_ctx* ctx, lagpm_box* box, double pfact);
  * cosmology. Returns when the step is complete; tree statistics and phase timings are filled.
  * Node arrays too small for the tree are grown and the tree kick and drift redone inside the call.
  * A tree walk whose bounded stack overflows returns LAGPM_E_OVERFLOW and leaves the box after the
- * drag and PM kick: no tree kick (FP32; the FP64 walk has kicked every other particle) and no
- * drift, so the positions are those the step started from. */
+ * drag and PM kick: no tree kick and no drift, so the positions are those the step started from
+ * (FP32; the FP64 walk's stack cannot overflow). */
 int lagpm_kdk_step(lagpm_ctx* ctx, lagpm_box* box, double anow, double astep);
 /* The same step for nbox independent boxes (box i at anow[i], astep[i]); no counterpart in
  * the reference, which evolves one box per MPI job. The boxes' PM phases and tree builds run

@@ -136,7 +136,7 @@ void free_box(lagpm_box* b) {
     dfree(b->nd_com); dfree(b->nd_q0); dfree(b->nd_q1); dfree(b->nd_d); dfree(b->cellroot); dfree(b->gflag);
     dfree(b->w_link); dfree(b->w_geo); dfree(b->w_q0); dfree(b->w_q1); dfree(b->w_rfc); dfree(b->w_cellroot);
     dfree(b->dep_scan_tmp); dfree(b->dep_blk);
-    dfree(b->goff); dfree(b->groups); dfree(b->gbox); dfree(b->pgroup); dfree(b->counters); dfree(b->dsz);
+    dfree(b->goff); dfree(b->groups); dfree(b->counters); dfree(b->dsz);
     dfree(b->scan_tmp);
 }
 
@@ -452,13 +452,13 @@ size_t lagpm_estimate_box_bytes(const lagpm_params* p, size_t np) {
     const int L = lagpm_choose_cell_level(p->n, p->rsphere);
     const size_t mcell = (size_t)1 << L;
     size_t b = (np + LAGPM_ARRAY_PAD) * 12 * 8 + np * (4 * 4 + 2 * 8 + 2 * 4);  // two sets of x..vz, id/id_alt/perm/perm2, keys, node counts
-    b += np * (f64 ? 4 : 16);                             // pgroup / pp
+    if (!f64) b += np * 16;                               // pp
     b += m * 8 + K * 2 * real + 4 * m * real;              // acc, padded FFT mesh, grad
     b += (f64 ? 4 : 8) * mcell * mcell * mcell + 4 * 8 + DSZ_COUNT * 4;  // cell roots, counters, sizes
     b += 4 * (lagpm_deposit_chunk_cap(p->n, np) + 1);     // deposit chunk starts
     b += 12 * (lagpm_deposit_blocks(p->n) + 1) + lagpm_scan_tmp_bytes(lagpm_deposit_blocks(p->n));  // chunk list
     const size_t cap = lagpm_tree_node_cap_guess(np, (int)mcell), gcap = cap + np / 64 + 1;
-    b += cap * (16 + 4 + 32 + 4 + 4 + (f64 ? 96 : 48 + 68)) + gcap * (8 + (f64 ? 48 : 0));  // (+ the FP32 walk's copy)
+    b += cap * (16 + 4 + 32 + 4 + 4 + (f64 ? 96 : 48 + 68)) + gcap * 8;  // (+ the FP32 walk's copy)
     b += std::max(lagpm_scan_tmp_bytes(cap), std::max(lagpm_scan_tmp_bytes(np), lagpm_sort_tmp_bytes(np)));
     return b;
 }
@@ -504,15 +504,14 @@ int lagpm_box_create(lagpm_ctx* ctx, const lagpm_params* p, size_t np, lagpm_box
     ALLOC(box->dep_blk, 3 * (nblk + 1));
     box->dep_cap = lagpm_deposit_chunk_cap(p->n, np) + 1;
     ALLOC(box->dep_start, box->dep_cap);
-    if (f64) ALLOC(box->pgroup, np);
-    else ALLOC(box->pp, np);
+    if (!f64) ALLOC(box->pp, np);
 #undef ALLOC
     if (rc == LAGPM_OK) {
         // node arrays and scan scratch (grown later if an input needs more nodes)
         rc = lagpm_tree_alloc(ctx, box, lagpm_tree_node_cap_guess(np, box->mcell));
         if (rc == LAGPM_OK) {
             box->bytes += box->scan_tmp_bytes + box->node_cap * (16 + 4 + 32 + 4 + 4 + (f64 ? 96 : 48)) +
-                          box->group_cap * (8 + (f64 ? 48 : 0));
+                          box->group_cap * 8;
             // the node arrays may grow later (dense input); the estimate is what admission uses
             box->bytes = std::max(box->bytes, lagpm_estimate_box_bytes(p, np));
         }

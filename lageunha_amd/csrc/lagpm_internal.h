@@ -109,10 +109,10 @@ enum {
     DSZ_SCRATCH = 4,  // scan totals nobody reads
     DSZ_DEEPER = 5,   // the build met a node to split at its depth limit (the tree is redone)
     DSZ_WALKOVF = 6,  // a walk stack overflowed: that step's drift is skipped (the error is returned)
+    DSZ_TICKET = 7,   // groups handed out by the FP64 walk beyond its waves' first ones
     DSZ_LVL = 8,
     DSZ_LOFF = DSZ_LVL + LAGPM_KEY_BITS + 1,
-    DSZ_LCUR = DSZ_LOFF + LAGPM_KEY_BITS + 1,
-    DSZ_COUNT = DSZ_LCUR + LAGPM_KEY_BITS + 1
+    DSZ_COUNT = DSZ_LOFF + LAGPM_KEY_BITS + 1
 };
 
 // A box's tree sizes and interaction counters, read back at the end of a step.
@@ -206,8 +206,6 @@ struct lagpm_box {
     uint32_t* goff = nullptr;
     size_t group_cap = 0;
     int2* groups = nullptr;       // begin, count
-    double* gbox = nullptr;       // FP64 group bbox: 6 per group
-    int* pgroup = nullptr;        // group of each particle (FP64 plain walk)
     uint32_t* dsz = nullptr;      // DSZ_* device sizes
     unsigned long long* counters = nullptr;  // [0]=n_pp [1]=n_pc [2]=walk stack overflow
     const law_tables* tab = nullptr;

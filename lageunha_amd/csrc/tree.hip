@@ -223,8 +223,8 @@ __global__ void gather_vel_kernel(gather_set g, const uint32_t* __restrict__ per
 }
 
 __device__ inline void tree_reset(int t, uint32_t* __restrict__ dsz, unsigned long long* __restrict__ counters) {
-    if (t == DSZ_NODES || t == DSZ_GROUPS || t == DSZ_OVERFLOW || t == DSZ_DEEPER || t == DSZ_WALKOVF) dsz[t] = 0u;
-    if ((t >= DSZ_LVL && t < DSZ_LOFF) || (t >= DSZ_LCUR && t < DSZ_COUNT)) dsz[t] = 0u;
+    if (t == DSZ_NODES || t == DSZ_GROUPS || t == DSZ_OVERFLOW || t == DSZ_DEEPER || t == DSZ_WALKOVF || t == DSZ_TICKET) dsz[t] = 0u;
+    if (t >= DSZ_LVL && t < DSZ_LOFF) dsz[t] = 0u;
     if (t < 4) counters[t] = 0ull;
 }
 
@@ -682,22 +682,6 @@ __global__ void group_write_kernel(uint32_t* __restrict__ dsz, size_t cap, size_
     uint32_t g = goff[v];
     group_pack(info[v], L, G, runs, info, child, parent, v, [&](int b, int m) { groups[g++] = make_int2(b, m); });
 }
-__global__ void group_box_kernel(const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ z,
-                                 const uint32_t* __restrict__ dsz, size_t gcap, const int2* __restrict__ groups,
-                                 double* __restrict__ gbox, int* __restrict__ pgroup) {
-    size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (dsz[DSZ_OVERFLOW] || g >= dev_count(dsz, DSZ_GROUPS, gcap)) return;
-    int2 gr = groups[g];
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (int p = gr.x; p < gr.x + gr.y; p++) {
-        lo[0] = fmin(lo[0], x[p]); hi[0] = fmax(hi[0], x[p]);
-        lo[1] = fmin(lo[1], y[p]); hi[1] = fmax(hi[1], y[p]);
-        lo[2] = fmin(lo[2], z[p]); hi[2] = fmax(hi[2], z[p]);
-        pgroup[p] = (int)g;
-    }
-    for (int a = 0; a < 3; a++) { gbox[6 * g + a] = lo[a]; gbox[6 * g + 3 + a] = hi[a]; }
-}
-
 // start of a tree build: clear the size words and the interaction counters (a kernel, not a
 // memset, so the step can be captured in a graph)
 __global__ void tree_reset_kernel(uint32_t* __restrict__ dsz, unsigned long long* __restrict__ counters) {
@@ -1369,159 +1353,354 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
     }
 }
 
-// Plain FP64 walk: one thread per target, private stack, same tree, groups and criteria.
+// FP64 walk: the same tree, groups and criteria in FP64 throughout, one wavefront per target group.
+// It was one thread per target, depth first, each on its own path: 64 lanes then read 64 nodes and
+// 64 leaves of their own, from L2, and table lines too (theta = 0.5: 32^3 2.95 ms, 64^3 6.2, 128^3
+// 26.3; this: 0.50, 1.37, 5.0). Now a wave pops up to 64 nodes of its group's stack at a time, one per lane, and its targets share
+// the accepted nodes and the listed sources: sources are staged in LDS 64 at a time (those beyond the
+// cutoff from the group's box dropped), the pair term's table lines (value and slope, 80 KB) are in
+// LDS, and lane (slot, rep) sums every R-th source for its M targets. 16 waves and one table fill a
+// CU's LDS. A team of 1 or 4 waves takes a group: each wave walks down the same way until the
+// stack holds enough nodes, then keeps every S-th of them (before that it takes every S-th of the
+// accepted nodes and leaves), and the team's sums meet in LDS in a fixed order.
+// What bounds it: FP64 issue in the pair loop (about 20 operations a pair) for large
+// boxes, the heaviest group's own time for small ones.
 struct walk64_args {
     const double *x, *y, *z;
-    double mass;
     const int4* info;
     const int* child;
     const double* nd;
     const int* cellroot;
     const uint64_t* key;
     int cell_shift;
-    const double* gbox;
-    const int* pgroup;
     const double* tab;
+    int nbins;
     float lam;
     double *vx, *vy, *vz;
     unsigned long long* counters;
-    uint32_t* dsz;
-    size_t np;
+    const uint32_t* dsz;
+    const int2* groups;
+    uint32_t* ticket;
+    int team;  // waves per group: 1 or 4
     int mcell;
-    double box, cellw, rc2, rcut, inv_theta2, fact;
+    double box, rc2, rcut, inv_theta2, fact;
     int naccept;
-    // sampled walk: target t is the particle at sample[t].x, opened as a group of its own (the
-    // per-particle test), its acceleration written to out[3t..3t+2] (velocities untouched)
-    const int2* sample;
+    // sampled walk: group g is the particle groups[g].x alone (the per-particle test), its
+    // acceleration written to out[3g..3g+2] (velocities untouched)
     double* out;
-    size_t nsample;
+    uint32_t nsample;
 };
 
-template <bool LOGT>
-// one target particle; returns false on a stack overflow (the kick is then not applied)
-__device__ inline bool walk_f64_target(const walk64_args& A, size_t i, unsigned long long& npp, unsigned long long& npc,
-                                       double* out) {
-    const double px0 = A.x[i], py0 = A.y[i], pz0 = A.z[i];
-    double lo[3] = {px0, py0, pz0}, hi[3] = {px0, py0, pz0};  // a group of one (sampled walk)
-    if (!out) {
-        const int g = A.pgroup[i];
-        for (int a = 0; a < 3; a++) {
-            lo[a] = A.gbox[6 * g + a];
-            hi[a] = A.gbox[6 * g + 3 + a];
-        }
-    }
-    // all group members share a chaining cell: the level-L prefix of their Morton key
-    const uint64_t cellkey = A.key[i] >> A.cell_shift;
-    const int cx = (int)compact3(cellkey), cy = (int)compact3(cellkey >> 1), cz = (int)compact3(cellkey >> 2);
-    int stack[256];
-    int sp = 0;
-    for (int nb = 26; nb >= 0; nb--) {
-        int dx = nb % 3 - 1, dy = (nb / 3) % 3 - 1, dz = nb / 9 - 1;
-        int nx = (cx + dx + A.mcell) % A.mcell, ny = (cy + dy + A.mcell) % A.mcell, nz = (cz + dz + A.mcell) % A.mcell;
-        int r = A.cellroot[nx + A.mcell * (ny + A.mcell * nz)];
-        if (r >= 0) stack[sp++] = (r << 5) | nb;
-    }
-    double ax = 0, ay = 0, az = 0;
-    bool overflow = false;
-    while (sp > 0) {
-        int e = stack[--sp];
-        int v = e >> 5, nb = e & 31;
-        int tx = cx + nb % 3 - 1, ty = cy + (nb / 3) % 3 - 1, tz = cz + nb / 9 - 1;
-        double sx = tx < 0 ? -A.box : (tx >= A.mcell ? A.box : 0.0);
-        double sy = ty < 0 ? -A.box : (ty >= A.mcell ? A.box : 0.0);
-        double sz = tz < 0 ? -A.box : (tz >= A.mcell ? A.box : 0.0);
-        const double* m = A.nd + 12 * (size_t)v;
-        int4 nd = A.info[v];
-        double qx = m[0] + sx, qy = m[1] + sy, qz = m[2] + sz, rmax = m[11];
-        double ddx = fmax(fmax(lo[0] - qx, qx - hi[0]), 0.0);
-        double ddy = fmax(fmax(lo[1] - qy, qy - hi[1]), 0.0);
-        double ddz = fmax(fmax(lo[2] - qz, qz - hi[2]), 0.0);
-        double dmin2 = ddx * ddx + ddy * ddy + ddz * ddz;
-        double rr = A.rcut + rmax;
-        if (dmin2 > rr * rr) continue;
-        if (nd.y >= A.naccept && dmin2 >= rmax * rmax * A.inv_theta2) {
-            npc++;
-            double dx = px0 - qx, dy = py0 - qy, dz = pz0 - qz;
-            double r2 = dx * dx + dy * dy + dz * dz;
-            if (r2 <= A.rc2) {
-                double t;
-                const int nt = table_bin64<LOGT>(r2, t, A.lam);
-                const double* tb = A.tab + 6 * nt;
-                double f1 = tb[0] + tb[1] * t, f2 = tb[2] + tb[3] * t, f3 = tb[4] + tb[5] * t;
-                double qx1 = m[4] * dx + m[7] * dy + m[8] * dz;
-                double qx2 = m[7] * dx + m[5] * dy + m[9] * dz;
-                double qx3 = m[8] * dx + m[9] * dy + m[6] * dz;
-                double qxy = m[4] * dx * dx + m[5] * dy * dy + m[6] * dz * dz + 2 * (m[7] * dx * dy + m[8] * dx * dz + m[9] * dy * dz);
-                double tmp = m[3] * f1 + m[10] * f2 + qxy * f3;
-                ax += dx * tmp + qx1 * 2 * f2;
-                ay += dy * tmp + qx2 * 2 * f2;
-                az += dz * tmp + qx3 * 2 * f2;
-            }
-        } else if (nd.z == 0) {
-            for (int p = nd.x; p < nd.x + nd.y; p++) {
-                npp++;
-                double dx = px0 - (A.x[p] + sx), dy = py0 - (A.y[p] + sy), dz = pz0 - (A.z[p] + sz);
-                double r2 = dx * dx + dy * dy + dz * dz;
-                if (r2 <= A.rc2) {
-                    double t;
-                    const int nt = table_bin64<LOGT>(r2, t, A.lam);
-                    double f = A.tab[6 * nt] + A.tab[6 * nt + 1] * t;  // unit particle mass
-                    ax += dx * f; ay += dy * f; az += dz * f;
-                }
-            }
-        } else {
-            if (sp + nd.z > 256) {
-                overflow = true;
-                break;
-            }
-            for (int c = nd.z - 1; c >= 0; c--) stack[sp++] = (A.child[8 * v + c] << 5) | nb;
-        }
-    }
-    if (overflow) return false;
-    if (out) {
-        out[0] = A.fact * ax;
-        out[1] = A.fact * ay;
-        out[2] = A.fact * az;
-        return true;
-    }
-    A.vx[i] += A.fact * ax;
-    A.vy[i] += A.fact * ay;
-    A.vz[i] += A.fact * az;
-    return true;
-}
-__device__ inline unsigned long long wave_sum_u64(unsigned long long v) {
+constexpr int W64_STACK = 512;  // stack entries per wave; a pop takes no more nodes than leave room for their children
+constexpr int W64_SLOTS = 2048;  // listed particles of one expansion (a bit each)
+
+__device__ inline double wave_min64(double v) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const unsigned lo = (unsigned)__shfl_xor((int)(unsigned)v, o, 64);
-        const unsigned hi = (unsigned)__shfl_xor((int)(unsigned)(v >> 32), o, 64);
-        v += ((unsigned long long)hi << 32) | lo;
-    }
+    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
     return v;
 }
-// Thread per target. The interaction counters are summed over the wave first: one atomic per
-// wave and counter (an atomic per thread on one address serialises millions of operations).
+__device__ inline double wave_max64(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
 template <bool LOGT>
-__global__ void __launch_bounds__(128) walk_f64_kernel(walk64_args A) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned long long npp = 0, npc = 0, ovf = 0;
-    if (!A.dsz[DSZ_OVERFLOW]) {
-        if (A.sample) {
-            if (t < A.nsample)
-                ovf = walk_f64_target<LOGT>(A, (size_t)A.sample[t].x, npp, npc, A.out + 3 * t) ? 0ull : 1ull;
-        } else if (t < A.np) {
-            ovf = walk_f64_target<LOGT>(A, t, npp, npc, nullptr) ? 0ull : 1ull;
+__global__ void __launch_bounds__(WALK_THREADS) walk_f64_kernel(walk64_args A) {
+    __shared__ double2 s_tab[TAB_LDS];  // value and slope of the pair term
+    __shared__ int s_stack[WALK_WAVES][W64_STACK];
+    __shared__ double s_src[WALK_WAVES][3][64];
+    __shared__ uint32_t s_head[WALK_WAVES][W64_SLOTS / 32];
+    __shared__ int2 s_leaf[WALK_WAVES][64];
+    __shared__ int s_pc[WALK_WAVES][64];
+    __shared__ uint32_t s_bar[WALK_WAVES], s_next[WALK_WAVES];  // per team: arrivals, next group
+    if (threadIdx.x < WALK_WAVES) s_bar[threadIdx.x] = 0u;
+    for (int i = threadIdx.x; i < A.nbins; i += WALK_THREADS) s_tab[i] = make_double2(A.tab[6 * i], A.tab[6 * i + 1]);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    int* stack = s_stack[wid];
+    double *sx = s_src[wid][0], *sy = s_src[wid][1], *sz = s_src[wid][2];
+    uint32_t* head = s_head[wid];
+    int2* leaf = s_leaf[wid];
+    int* pcl = s_pc[wid];
+    const uint32_t ngroups = A.dsz[DSZ_OVERFLOW] ? 0u : (A.out ? A.nsample : A.dsz[DSZ_GROUPS]);
+    const int S = A.team, team = wid / S, part = wid & (S - 1);
+    const uint32_t nteams = gridDim.x * (uint32_t)(WALK_WAVES / S);
+    uint32_t arrived = 0;
+    // All waves of the team have written their LDS when it returns. Every wave of a team takes the
+    // same groups and so as many of these waits as the others, and all are resident: each ends.
+    auto team_sync = [&]() {
+        wave_sync();
+        if (S == 1) return;
+        arrived += (uint32_t)S;
+        if (lane == 0) {
+            __hip_atomic_fetch_add(&s_bar[team], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            while (__hip_atomic_load(&s_bar[team], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < arrived) __builtin_amdgcn_s_sleep(1);
         }
+        wave_sync();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+    const double rc2_keep = A.rc2 * (1.0 + 1e-12);  // a source beyond it from the group's box adds exactly zero
+    unsigned long long npp = 0, npc = 0;
+    // the first group by rank (the teams of one CU far apart: few groups spread over all CUs), the
+    // others by ticket (see the FP32 walk)
+    for (uint32_t g = (uint32_t)team * gridDim.x + blockIdx.x; g < ngroups;) {
+        const int2 gr = A.groups[g];
+        const int gbeg = __builtin_amdgcn_readfirstlane(gr.x), cnt = __builtin_amdgcn_readfirstlane(gr.y);
+        // lanes (slot, rep): slots x R of them, M targets each; three targets a lane where that uses
+        // at least as many lanes, and for groups of more than 64
+        const int s3 = (cnt + 2) / 3, R3 = 64 / s3, R1 = cnt <= 64 ? 64 / cnt : 0;
+        auto group_body = [&](auto mc) {
+            constexpr int M = decltype(mc)::value;
+            const int slots = M == 3 ? s3 : cnt, R = M == 3 ? R3 : R1;
+            const int rep = lane / slots, slot = lane - rep * slots;
+            const bool act = rep < R;
+            double xt[M], yt[M], zt[M], ax[M], ay[M], az[M];
+            int me[M];
+            bool valid[M];
+            double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+#pragma unroll
+            for (int i = 0; i < M; i++) {
+                const int t = slot + i * slots;
+                valid[i] = act && t < cnt;
+                me[i] = gbeg + (valid[i] ? t : 0);  // an idle lane repeats target 0: inside the group's box
+                xt[i] = A.x[me[i]]; yt[i] = A.y[me[i]]; zt[i] = A.z[me[i]];
+                ax[i] = ay[i] = az[i] = 0.0;
+                lo[0] = fmin(lo[0], xt[i]); hi[0] = fmax(hi[0], xt[i]);
+                lo[1] = fmin(lo[1], yt[i]); hi[1] = fmax(hi[1], yt[i]);
+                lo[2] = fmin(lo[2], zt[i]); hi[2] = fmax(hi[2], zt[i]);
+            }
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                lo[a] = wave_min64(lo[a]);
+                hi[a] = wave_max64(hi[a]);
+            }
+            // all group members share a chaining cell: the level-L prefix of their Morton key
+            const uint64_t cellkey = A.key[gbeg] >> A.cell_shift;
+            const int cx = (int)compact3(cellkey), cy = (int)compact3(cellkey >> 1), cz = (int)compact3(cellkey >> 2);
+            auto shift_of = [&](int nb, double& qx, double& qy, double& qz) {
+                const int tx = cx + nb % 3 - 1, ty = cy + (nb / 3) % 3 - 1, tz = cz + nb / 9 - 1;
+                qx = tx < 0 ? -A.box : (tx >= A.mcell ? A.box : 0.0);
+                qy = ty < 0 ? -A.box : (ty >= A.mcell ? A.box : 0.0);
+                qz = tz < 0 ? -A.box : (tz >= A.mcell ? A.box : 0.0);
+            };
+            auto box_dist2 = [&](double qx, double qy, double qz) {
+                const double ddx = fmax(fmax(lo[0] - qx, qx - hi[0]), 0.0);
+                const double ddy = fmax(fmax(lo[1] - qy, qy - hi[1]), 0.0);
+                const double ddz = fmax(fmax(lo[2] - qz, qz - hi[2]), 0.0);
+                return ddx * ddx + ddy * ddy + ddz * ddz;
+            };
+            int sp = 0;
+            {
+                int e = -1;
+                if (lane < 27) {
+                    const int dx = lane % 3 - 1, dy = (lane / 3) % 3 - 1, dz = lane / 9 - 1;
+                    const int nx = (cx + dx + A.mcell) % A.mcell, ny = (cy + dy + A.mcell) % A.mcell, nz = (cz + dz + A.mcell) % A.mcell;
+                    const int r = A.cellroot[nx + A.mcell * (ny + A.mcell * nz)];
+                    if (r >= 0) e = (r << 5) | lane;
+                }
+                const int off = wave_excl_count(e >= 0, sp);
+                if (e >= 0) stack[off] = e;
+                wave_sync();
+            }
+            bool split = S == 1;  // the stack holds this wave's share alone
+            int fill = 0;  // staged sources, wave-uniform
+            auto pp_chunk = [&](int m) {
+                if (!act) return;
+                for (int k = rep; k < m; k += R) {
+                    const double qx = sx[k], qy = sy[k], qz = sz[k];
+#pragma unroll
+                    for (int i = 0; i < M; i++) {
+                        const double dx = xt[i] - qx, dy = yt[i] - qy, dz = zt[i] - qz;
+                        const double r2 = dx * dx + dy * dy + dz * dz;
+                        double t;
+                        const double2 tb = s_tab[table_bin64<LOGT>(r2, t, A.lam)];
+                        const double f = r2 <= A.rc2 ? tb.x + tb.y * t : 0.0;  // unit particle mass
+                        ax[i] += dx * f; ay[i] += dy * f; az[i] += dz * f;
+                    }
+                }
+            };
+            // particles of 64 slots (in: this lane's slot holds one), those near the group to the chunk
+            auto stage = [&](bool in, int p, int nb) {
+                double qx = 0.0, qy = 0.0, qz = 0.0;
+                if (in) {
+                    double hx, hy, hz;
+                    shift_of(nb, hx, hy, hz);
+                    qx = A.x[p] + hx; qy = A.y[p] + hy; qz = A.z[p] + hz;
+                }
+                const bool keep = in && box_dist2(qx, qy, qz) <= rc2_keep;
+                int tot;
+                const int off = wave_excl_count(keep, tot);
+                const int room = 64 - fill;
+                if (keep && off < room) { sx[fill + off] = qx; sy[fill + off] = qy; sz[fill + off] = qz; }
+                fill += tot;
+                wave_sync();
+                if (fill >= 64) {
+                    pp_chunk(64);
+                    wave_sync();
+                    if (keep && off >= room) { sx[off - room] = qx; sy[off - room] = qy; sz[off - room] = qz; }
+                    fill -= 64;
+                    wave_sync();
+                }
+            };
+            // the particles of the lanes' leaves (first particle, count; count 0: none): slot s of an
+            // expansion belongs to the last leaf whose first slot is not after it, found by counting
+            // the marks of first slots
+            auto leaves = [&](int first, int count, int nb) {
+                for (int done = 0; done < 64;) {
+                    int all;
+                    const int c = lane >= done ? min(count, W64_SLOTS + 1) : 0;
+                    const int P = wave_excl_scan(c, lane, all);
+                    if (all == 0) break;
+                    // lanes done .. m - 1 fit (a prefix); none: lane `done` alone holds more than the marks cover
+                    const int m = __builtin_amdgcn_readfirstlane(__popcll(__ballot(P + c <= W64_SLOTS)));
+                    if (m <= done) {
+                        const int b0 = __builtin_amdgcn_readlane(first, done), n0 = __builtin_amdgcn_readlane(count, done);
+                        const int nb0 = __builtin_amdgcn_readlane(nb, done);
+                        npp += (unsigned long long)n0 * (unsigned)cnt;
+                        for (int s = 0; s < n0; s += 64) stage(s + lane < n0, b0 + s + lane, nb0);
+                        done++;
+                        continue;
+                    }
+                    const int T = __builtin_amdgcn_readlane(P + c, m - 1);
+                    npp += (unsigned long long)T * (unsigned)cnt;
+                    if (32 * lane < T) head[lane] = 0u;
+                    wave_sync();
+                    int held;
+                    const bool has = lane >= done && lane < m && c > 0;
+                    const int k = wave_excl_count(has, held);
+                    if (has) {
+                        atomicOr(&head[P >> 5], 1u << (P & 31));
+                        leaf[k] = make_int2(first - P, nb);
+                    }
+                    wave_sync();
+                    int before = -1;
+                    for (int s0 = 0; s0 < T; s0 += 64) {
+                        const unsigned wl = (unsigned)__builtin_amdgcn_readfirstlane((int)head[s0 >> 5]);
+                        const unsigned wh = (unsigned)__builtin_amdgcn_readfirstlane((int)head[(s0 >> 5) + 1]);
+                        const unsigned long long w = ((unsigned long long)wh << 32) | wl, w1 = w >> 1;
+                        const int j = before + (int)(wl & 1u) +
+                                      (int)__builtin_amdgcn_mbcnt_hi((unsigned)(w1 >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)w1, 0u));
+                        before += __popcll(w);
+                        const bool in = s0 + lane < T;
+                        const int2 e = leaf[in ? j : 0];
+                        stage(in, e.x + s0 + lane, e.y);
+                    }
+                    done = m;
+                }
+            };
+            while (sp > 0) {
+                // after a pop of `take` nodes at most 7 take more entries: kept below the stack's end
+                // less 128; a single node at a time always fits (7 more entries a level, 14 levels)
+                const int take = min(min(sp, 64), max(1, (W64_STACK - 128 - sp) / 7));
+                sp -= take;
+                const int e = lane < take ? stack[sp + lane] : -1;
+                wave_sync();
+                int kind = 0;  // 0 none, 1 accept, 2 leaf, 3 open
+                int4 nd = make_int4(0, 0, 0, 0);
+                int v = 0, nb = 0;
+                if (e >= 0) {
+                    v = e >> 5;
+                    nb = e & 31;
+                    double hx, hy, hz;
+                    shift_of(nb, hx, hy, hz);
+                    const double* m = A.nd + 12 * (size_t)v;
+                    nd = A.info[v];
+                    const double rmax = m[11];
+                    const double dmin2 = box_dist2(m[0] + hx, m[1] + hy, m[2] + hz);
+                    const double rr = A.rcut + rmax;
+                    if (dmin2 > rr * rr) kind = 0;
+                    else if (nd.y >= A.naccept && dmin2 >= rmax * rmax * A.inv_theta2) kind = 1;
+                    else kind = nd.z == 0 ? 2 : 3;
+                }
+                int tot;
+                const int nch = kind == 3 ? nd.z : 0;
+                const int off = wave_excl_scan(nch, lane, tot);
+                for (int c = 0; c < nch; c++) stack[sp + off + c] = (A.child[8 * (size_t)v + c] << 5) | nb;
+                sp += tot;
+                wave_sync();
+                if (!split && (lane & (S - 1)) != part) kind = 0;  // another wave's
+                if (!split && sp >= 16 * S) {
+                    const int n = (sp - part + S - 1) / S;
+                    for (int k = 0; k < n; k += 64) {  // (entries move towards the bottom: read, then written)
+                        const int q = k + lane < n ? stack[(k + lane) * S + part] : 0;
+                        wave_sync();
+                        if (k + lane < n) stack[k + lane] = q;
+                        wave_sync();
+                    }
+                    sp = n;
+                    split = true;
+                }
+                int nacc;
+                const int poff = wave_excl_count(kind == 1, nacc);
+                if (kind == 1) pcl[poff] = e;
+                wave_sync();
+                npc += (unsigned long long)nacc * (unsigned)cnt;
+                if (act) {
+                    for (int k = rep; k < nacc; k += R) {
+                        const int q = pcl[k];
+                        double hx, hy, hz;
+                        shift_of(q & 31, hx, hy, hz);
+                        const double* m = A.nd + 12 * (size_t)(q >> 5);
+                        const double qx = m[0] + hx, qy = m[1] + hy, qz = m[2] + hz;
+#pragma unroll
+                        for (int i = 0; i < M; i++) {
+                            const double dx = xt[i] - qx, dy = yt[i] - qy, dz = zt[i] - qz;
+                            const double r2 = dx * dx + dy * dy + dz * dz;
+                            if (r2 > A.rc2) continue;
+                            double t;
+                            const double* tb = A.tab + 6 * table_bin64<LOGT>(r2, t, A.lam);
+                            const double f1 = tb[0] + tb[1] * t, f2 = tb[2] + tb[3] * t, f3 = tb[4] + tb[5] * t;
+                            const double qx1 = m[4] * dx + m[7] * dy + m[8] * dz;
+                            const double qx2 = m[7] * dx + m[5] * dy + m[9] * dz;
+                            const double qx3 = m[8] * dx + m[9] * dy + m[6] * dz;
+                            const double qxy = dx * qx1 + dy * qx2 + dz * qx3;
+                            const double tmp = m[3] * f1 + m[10] * f2 + qxy * f3;
+                            ax[i] += dx * tmp + qx1 * 2 * f2;
+                            ay[i] += dy * tmp + qx2 * 2 * f2;
+                            az[i] += dz * tmp + qx3 * 2 * f2;
+                        }
+                    }
+                }
+                leaves(nd.x, kind == 2 ? nd.y : 0, nb);
+            }
+            if (fill > 0) pp_chunk(fill);
+            wave_sync();
+            // the R partial sums of each target in each of the team's waves, in a fixed order (the
+            // chunk's LDS is free now); the team's first wave adds them up and takes the next group
+            if (part == 0 && lane == 0) s_next[team] = nteams + atomicAdd(A.ticket, 1u);
+#pragma unroll
+            for (int i = 0; i < M; i++) {
+                sx[lane] = ax[i]; sy[lane] = ay[i]; sz[lane] = az[i];
+                team_sync();
+                if (part == 0 && rep == 0 && valid[i]) {
+                    double fx = 0.0, fy = 0.0, fz = 0.0;
+                    for (int w = 0; w < S; w++)
+                        for (int r = 0; r < R; r++) {
+                            fx += s_src[wid + w][0][slot + r * slots];
+                            fy += s_src[wid + w][1][slot + r * slots];
+                            fz += s_src[wid + w][2][slot + r * slots];
+                        }
+                    if (A.out) {
+                        A.out[3 * (size_t)g] = A.fact * fx;
+                        A.out[3 * (size_t)g + 1] = A.fact * fy;
+                        A.out[3 * (size_t)g + 2] = A.fact * fz;
+                    } else {
+                        A.vx[me[i]] += A.fact * fx;
+                        A.vy[me[i]] += A.fact * fy;
+                        A.vz[me[i]] += A.fact * fz;
+                    }
+                }
+                team_sync();
+            }
+        };
+        if (R3 >= 3 * R1) group_body(ic<3>{});
+        else group_body(ic<1>{});
+        g = (uint32_t)__builtin_amdgcn_readfirstlane((int)*(volatile uint32_t*)&s_next[team]);
     }
-    npp = wave_sum_u64(npp);
-    npc = wave_sum_u64(npc);
-    ovf = wave_sum_u64(ovf);
-    if ((threadIdx.x & 63) == 0) {
-        if (npp) atomicAdd(&A.counters[0], npp);
-        if (npc) atomicAdd(&A.counters[1], npc);
-        if (ovf) {
-            atomicAdd(&A.counters[2], ovf);
-            atomicOr(&A.dsz[DSZ_WALKOVF], 1u);
-        }
+    if (lane == 0 && (npp | npc)) {
+        atomicAdd(&A.counters[0], npp);
+        atomicAdd(&A.counters[1], npc);
     }
 }
 
@@ -1570,7 +1749,6 @@ int lagpm_tree_alloc(lagpm_ctx* ctx, lagpm_box* box, size_t cap) {
     RCHK(regrow(ctx, &box->groups, gcap));
     if (f64) {
         RCHK(regrow(ctx, &box->nd_d, 12 * cap));
-        RCHK(regrow(ctx, &box->gbox, 6 * gcap));
     } else {
         RCHK(regrow(ctx, &box->nd_com, cap));
         RCHK(regrow(ctx, &box->nd_q0, cap));
@@ -1717,11 +1895,6 @@ int lagpm_tree_build(lagpm_ctx* ctx, lagpm_box* box) {
     hipLaunchKernelGGL(group_write_kernel, dim3(blocks_for(cap, 256)), dim3(256), 0, st, box->dsz, cap, gcap, L, G, runs,
                        box->nd_info, box->nd_child, box->nd_parent, box->gflag, box->goff, box->groups);
     HIPCHK(ctx, hipGetLastError());
-    if (f64) {
-        hipLaunchKernelGGL(group_box_kernel, dim3(blocks_for(gcap, 256)), dim3(256), 0, st, box->x, box->y, box->z,
-                           box->dsz, gcap, box->groups, box->gbox, box->pgroup);
-        HIPCHK(ctx, hipGetLastError());
-    }
     box->tree_built = true;
     return LAGPM_OK;
 }
@@ -1785,26 +1958,30 @@ int lagpm_tree_walk_f32(lagpm_ctx* ctx, lagpm_box* const* boxes, const double* f
 }
 
 int lagpm_tree_walk_f64(lagpm_ctx* ctx, lagpm_box* box, double fact, const walk_sample* sample) {
+    if (box->np == 0) return LAGPM_OK;
     const double th = box->p.theta;
-    const double cellw = (double)box->p.n / (double)box->mcell;
     walk64_args A;
-    A.x = box->x; A.y = box->y; A.z = box->z; A.mass = box->p.mass; A.info = box->nd_info; A.child = box->nd_child;
-    A.nd = box->nd_d; A.cellroot = box->cellroot; A.gbox = box->gbox;
-    A.key = box->key; A.cell_shift = 3 * (LAGPM_KEY_BITS - box->level_cell); A.pgroup = box->pgroup; A.tab = box->tab->tabd;
-    A.vx = box->vx; A.vy = box->vy; A.vz = box->vz; A.counters = box->counters; A.dsz = box->dsz; A.np = box->np;
-    A.mcell = box->mcell; A.box = (double)box->p.n; A.cellw = cellw; A.rc2 = box->tab->rc2_eff; A.lam = box->tab->lam;
+    A.x = box->x; A.y = box->y; A.z = box->z; A.info = box->nd_info; A.child = box->nd_child;
+    A.nd = box->nd_d; A.cellroot = box->cellroot;
+    A.key = box->key; A.cell_shift = 3 * (LAGPM_KEY_BITS - box->level_cell);
+    A.tab = box->tab->tabd; A.nbins = box->tab->nbins; A.lam = box->tab->lam;
+    A.vx = box->vx; A.vy = box->vy; A.vz = box->vz; A.counters = box->counters; A.dsz = box->dsz;
+    A.groups = sample ? sample->groups : box->groups;
+    A.ticket = (sample ? sample->dsz : box->dsz) + DSZ_TICKET;
+    A.mcell = box->mcell; A.box = (double)box->p.n; A.rc2 = box->tab->rc2_eff;
     A.rcut = box->p.rsphere; A.inv_theta2 = th > 0 ? 1.0 / (th * th) : 1e30;
     A.fact = fact * box->p.mass / ((double)box->p.n * (double)box->p.n);
     A.naccept = LAGPM_NACCEPT;
-    A.sample = sample ? sample->groups : nullptr;
     A.out = sample ? sample->out : nullptr;
-    A.nsample = sample ? sample->count : 0;
-    if (box->np == 0) return LAGPM_OK;
-    const size_t nthreads = sample ? sample->count : box->np;
-    if (box->tab->logr2)
-        hipLaunchKernelGGL(walk_f64_kernel<true>, dim3(blocks_for(nthreads, 128)), dim3(128), 0, box->st, A);
-    else
-        hipLaunchKernelGGL(walk_f64_kernel<false>, dim3(blocks_for(nthreads, 128)), dim3(128), 0, box->st, A);
+    A.nsample = sample ? (uint32_t)sample->count : 0u;
+    // Teams of four while a CU's waves get about two groups or less each: then the heaviest group's
+    // own time is the walk's. Walk in ms with one wave and with four: 32^3 0.56 and 0.50, 64^3 1.81 and
+    // 1.37, 72^3 (373,248 targets) 1.27 and 1.59, 96^3 2.3 and 3.0 (four waves each walk down to the split).
+    const size_t targets = sample ? 44 * sample->count : box->np;
+    A.team = targets <= 300000 ? 4 : 1;
+    const unsigned blocks = (unsigned)std::max(1, ctx->num_cu);  // one workgroup per CU (its LDS)
+    auto kern = box->tab->logr2 ? walk_f64_kernel<true> : walk_f64_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(WALK_THREADS), 0, box->st, A);
     HIPCHK(ctx, hipGetLastError());
     return LAGPM_OK;
 }
@@ -1891,7 +2068,7 @@ __global__ void sample_groups_kernel(const uint32_t* __restrict__ id, size_t np,
 }
 // the sample's size words: the box's (its overflow flag) with the group count replaced
 __global__ void sample_dsz_kernel(const uint32_t* __restrict__ dsz, uint32_t* __restrict__ sdsz, uint32_t count) {
-    for (int i = threadIdx.x; i < DSZ_COUNT; i += blockDim.x) sdsz[i] = i == DSZ_GROUPS ? count : dsz[i];
+    for (int i = threadIdx.x; i < DSZ_COUNT; i += blockDim.x) sdsz[i] = i == DSZ_GROUPS ? count : (i == DSZ_TICKET ? 0u : dsz[i]);
 }
 __global__ void sample_gather_kernel(const int2* __restrict__ groups, size_t count, const double* __restrict__ tx,
                                      const double* __restrict__ ty, const double* __restrict__ tz, double* __restrict__ out) {
