@@ -831,13 +831,15 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
     // one L2; a single global ticket would spread neighbours over all eight caches. An XCD that
     // has finished its range takes tickets from the next ranges in turn (work stealing), and a
     // wave leaves after finding all eight ranges exhausted.
-    // A wave's first group of its own range is its rank there, without an atomic, and later ones
+    // A wave's first group of its own range is its rank there (the waves of one workgroup far apart, so
+    // that few groups spread over all CUs), without an atomic, and later ones
     // come from the range's counter, each counter in a cache line of its own. Once a range is found
     // exhausted the workgroup's other waves skip it, and a range that the ranks alone cover is never
     // asked for. Device-wide atomics on one line are served one after another: when every wave
     // began with one and left by asking all eight ranges (of a 32^3 box's 741 groups: 33,000
     // atomics for 4096 waves), their queue also held up the first loads of the waves that had a
-    // group, by 0.2 ms of its 0.63 ms walk. Walk times before and after: 32^3 0.63 -> 0.41 ms, 64^3
+    // group, by 0.2 ms of its 0.63 ms walk, and 0.1 more went when 16 waves of a CU no
+    // longer began with neighbouring groups (first come had spread them). Walk times before and after: 32^3 0.63 -> 0.30 ms, 64^3
     // 0.75 -> 0.59, 100^3 1.47 -> 1.30, 128^3 2.14 -> 1.91, 256^3 13.94 -> 13.75.
     auto range_lo = [&](int x) -> int { return (int)(((long long)gtotal * x) / WALK_XCDS); };
     auto range_waves = [&](int x) -> int { return (((int)gridDim.x - x + WALK_XCDS - 1) / WALK_XCDS) * WALK_WAVES; };
@@ -849,7 +851,7 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
         const int lo = range_lo(slot), left = range_lo(slot + 1) - lo, ranked = range_waves(slot);
         int t = left;
         if (tries < 0) {
-            t = (int)(blockIdx.x / WALK_XCDS) * WALK_WAVES + __builtin_amdgcn_readfirstlane(wid);
+            t = __builtin_amdgcn_readfirstlane(wid) * (ranked / WALK_WAVES) + (int)(blockIdx.x / WALK_XCDS);
             tries = 0;
         } else if (left > ranked && !((__builtin_amdgcn_readfirstlane((int)*(volatile unsigned*)&s_done) >> slot) & 1)) {
             // Group ticket: one atomic per group, from lane 0 (an atomic executed by all 64 lanes is
