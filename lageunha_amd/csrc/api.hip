@@ -132,11 +132,10 @@ void free_box(lagpm_box* b) {
     lagpm_box_graphs_release(b);
     dfree(b->acc); dfree(b->dep_start); dfree(b->rho); dfree(b->grad);
     b->spec = b->phi = nullptr;  // the same padded mesh as rho
-    dfree(b->pp); dfree(b->ncount); dfree(b->noff); dfree(b->nd_info); dfree(b->nd_parent); dfree(b->nd_child);
-    dfree(b->nd_com); dfree(b->nd_q0); dfree(b->nd_q1); dfree(b->nd_d); dfree(b->cellroot); dfree(b->gflag);
-    dfree(b->w_link); dfree(b->w_geo); dfree(b->w_q0); dfree(b->w_q1); dfree(b->w_rfc); dfree(b->w_cellroot);
+    dfree(b->pp); dfree(b->nd_link); dfree(b->nd_lev); dfree(b->nd_rop); dfree(b->nd_geo); dfree(b->nd_q0); dfree(b->nd_q1);
+    dfree(b->nd_d); dfree(b->cellroot);
     dfree(b->dep_scan_tmp); dfree(b->dep_blk);
-    dfree(b->goff); dfree(b->groups); dfree(b->counters); dfree(b->dsz);
+    dfree(b->groups); dfree(b->counters); dfree(b->dsz);
     dfree(b->scan_tmp);
 }
 
@@ -451,15 +450,15 @@ size_t lagpm_estimate_box_bytes(const lagpm_params* p, size_t np) {
     const size_t real = f64 ? 8 : 4;
     const int L = lagpm_choose_cell_level(p->n, p->rsphere);
     const size_t mcell = (size_t)1 << L;
-    size_t b = (np + LAGPM_ARRAY_PAD) * 12 * 8 + np * (4 * 4 + 2 * 8 + 2 * 4);  // two sets of x..vz, id/id_alt/perm/perm2, keys, node counts
+    size_t b = (np + LAGPM_ARRAY_PAD) * 12 * 8 + np * (4 * 4 + 2 * 8);  // two sets of x..vz, id/id_alt/perm/perm2, keys
     if (!f64) b += np * 16;                               // pp
     b += m * 8 + K * 2 * real + 4 * m * real;              // acc, padded FFT mesh, grad
-    b += (f64 ? 4 : 8) * mcell * mcell * mcell + 4 * 8 + DSZ_COUNT * 4;  // cell roots, counters, sizes
+    b += 4 * mcell * mcell * mcell + 4 * 8 + DSZ_COUNT * 4;  // cell roots, counters, sizes
     b += 4 * (lagpm_deposit_chunk_cap(p->n, np) + 1);     // deposit chunk starts
     b += 12 * (lagpm_deposit_blocks(p->n) + 1) + lagpm_scan_tmp_bytes(lagpm_deposit_blocks(p->n));  // chunk list
     const size_t cap = lagpm_tree_node_cap_guess(np, (int)mcell), gcap = cap + np / 64 + 1;
-    b += cap * (16 + 4 + 32 + 4 + 4 + (f64 ? 96 : 48 + 68)) + gcap * 8;  // (+ the FP32 walk's copy)
-    b += std::max(lagpm_scan_tmp_bytes(cap), std::max(lagpm_scan_tmp_bytes(np), lagpm_sort_tmp_bytes(np)));
+    b += cap * (16 + 4 + 4 + (f64 ? 96 : 48)) + gcap * 8;
+    b += std::max(lagpm_tree_tmp_bytes(np, cap), lagpm_sort_tmp_bytes(np));
     return b;
 }
 
@@ -494,9 +493,7 @@ int lagpm_box_create(lagpm_ctx* ctx, const lagpm_params* p, size_t np, lagpm_box
     if (rc == LAGPM_OK) rc = dalloc(ctx, box, (char**)&box->rho, K * 2 * real);
     box->spec = box->phi = box->rho;
     if (rc == LAGPM_OK) rc = dalloc(ctx, box, (char**)&box->grad, m * 4 * real);
-    ALLOC(box->ncount, np); ALLOC(box->noff, np);
     ALLOC(box->cellroot, (size_t)box->mcell * box->mcell * box->mcell);
-    if (!f64) ALLOC(box->w_cellroot, (size_t)box->mcell * box->mcell * box->mcell);
     ALLOC(box->counters, 4);
     ALLOC(box->dsz, DSZ_COUNT);
     const size_t nblk = lagpm_deposit_blocks(p->n);
@@ -510,7 +507,7 @@ int lagpm_box_create(lagpm_ctx* ctx, const lagpm_params* p, size_t np, lagpm_box
         // node arrays and scan scratch (grown later if an input needs more nodes)
         rc = lagpm_tree_alloc(ctx, box, lagpm_tree_node_cap_guess(np, box->mcell));
         if (rc == LAGPM_OK) {
-            box->bytes += box->scan_tmp_bytes + box->node_cap * (16 + 4 + 32 + 4 + 4 + (f64 ? 96 : 48)) +
+            box->bytes += box->scan_tmp_bytes + box->node_cap * (16 + 4 + 4 + (f64 ? 96 : 48)) +
                           box->group_cap * 8;
             // the node arrays may grow later (dense input); the estimate is what admission uses
             box->bytes = std::max(box->bytes, lagpm_estimate_box_bytes(p, np));

@@ -106,7 +106,6 @@ enum {
     DSZ_GROUPS = 1,
     DSZ_CHUNKS = 2,
     DSZ_OVERFLOW = 3,
-    DSZ_SCRATCH = 4,  // scan totals nobody reads
     DSZ_DEEPER = 5,   // the build met a node to split at its depth limit (the tree is redone)
     DSZ_WALKOVF = 6,  // a walk stack overflowed: that step's drift is skipped (the error is returned)
     DSZ_TICKET = 7,   // groups handed out by the FP64 walk beyond its waves' first ones
@@ -181,29 +180,19 @@ struct lagpm_box {
     int level_cell = 0;       // chaining level L: 2^L cells per axis, width n/2^L >= rsphere
     int mcell = 0;            // 2^L
     float4* pp = nullptr;     // sorted FP32 positions + mass
-    uint32_t* ncount = nullptr;   // per-particle node count, then offsets
-    uint32_t* noff = nullptr;
     size_t node_cap = 0;          // capacity of the node arrays (device count may not exceed it)
-    int4* nd_info = nullptr;      // begin, count, nchild, level
-    int* nd_parent = nullptr;
-    int* nd_child = nullptr;      // 8 per node
-    float4* nd_com = nullptr;     // com.xyz, mass
-    float4* nd_q0 = nullptr;      // Qxx Qyy Qzz Qxy
-    float4* nd_q1 = nullptr;      // Qxz Qyz trQ rmax
-    double* nd_d = nullptr;       // FP64 moments: 12 per node (com3, mass, Q6, trQ, rmax)
-    int* cellroot = nullptr;      // mcell^3
-    // The FP32 walk's copy of the tree by record (the build's order: level by level, the children of
-    // a node consecutive): links (first particle, count, first child record, children), the opening
-    // test's geometry (com, rmax), the quadrupole (q0; q1 with the mass in place of rmax), the split's
-    // first child record of each record, and the cell roots as records (mcell^3).
-    int4* w_link = nullptr;
-    float4* w_geo = nullptr;
-    float4* w_q0 = nullptr;
-    float4* w_q1 = nullptr;
-    int* w_rfc = nullptr;
-    int* w_cellroot = nullptr;
-    uint32_t* gflag = nullptr;    // per-node group count, then offsets
-    uint32_t* goff = nullptr;
+    // The tree by record: level by level, in particle order within a level, the children of a node
+    // consecutive. Links (first particle, count, first child record or 0, children); level (bit 8: first
+    // child of its parent); the record of each pre-order number. FP32: centre and rmax, quadrupole (q0: xx
+    // yy zz xy; q1: xz yz, half the trace, mass). FP64: 12 doubles (com3, mass, Q6, trQ, rmax).
+    int4* nd_link = nullptr;
+    int* nd_lev = nullptr;
+    uint32_t* nd_rop = nullptr;
+    float4* nd_geo = nullptr;
+    float4* nd_q0 = nullptr;
+    float4* nd_q1 = nullptr;
+    double* nd_d = nullptr;
+    int* cellroot = nullptr;      // root record of each chaining cell or -1 (mcell^3)
     size_t group_cap = 0;
     int2* groups = nullptr;       // begin, count
     uint32_t* dsz = nullptr;      // DSZ_* device sizes
@@ -320,6 +309,7 @@ int lagpm_tree_finish_with(lagpm_ctx* ctx, lagpm_box* box, const tree_readback& 
 int lagpm_tree_alloc(lagpm_ctx* ctx, lagpm_box* box, size_t node_cap);
 double lagpm_tree_scale(const lagpm_box* box);  // FP32 tree coordinate scale (sqrt(lam) or 1)
 size_t lagpm_tree_node_cap_guess(size_t np, int mcell);
+size_t lagpm_tree_tmp_bytes(size_t np, size_t cap);  // scratch of a build of np particles into cap nodes
 int lagpm_choose_cell_level(int n, double rsphere);
 size_t lagpm_walk_stack_entries(int num_cu);
 

@@ -982,8 +982,7 @@ int lagpm_pm_deposit(lagpm_ctx* ctx, lagpm_box* box) {
     } else {
         // chunk list from the sorted keys (the caller sorted the particles); the chunk count
         // stays on the device and the deposit grid covers its upper bound. Its scratch is its own
-        // (dep_blk, dep_scan_tmp): a step runs the deposit beside the tree build, which uses
-        // ncount, noff and scan_tmp.
+        // (dep_blk, dep_scan_tmp): a step runs the deposit beside the tree build, which uses scan_tmp.
         const int lvl = deposit_block_level(n);
         const int sh = 3 * (LAGPM_KEY_BITS - lvl);
         const uint32_t nblk = (uint32_t)lagpm_deposit_blocks(n);

@@ -228,29 +228,6 @@ __device__ inline void tree_reset(int t, uint32_t* __restrict__ dsz, unsigned lo
     if (t < 4) counters[t] = 0ull;
 }
 
-// Everything the build needs cleared or packed before the level-L cells, in one pass: the build's
-// sizes and counters, per-particle node counts, empty cell roots, and (FP32 tree, pp non-null)
-// the pp copy of the positions in units of the particle mass.
-// pp is the FP32 copy of the positions for the tree, scaled by sc (rounded once from the FP64
-// product): with the log-r^2 force tables sc = sqrt(lam), so a pair's r^2 in these units is lam r^2,
-// the table variable, and needs no multiply in the pair loop. Everything the FP32 tree derives
-// from pp (centres, second moments, node sizes, group boxes) is in the same units.
-__global__ void tree_prep_kernel(const double* __restrict__ x, const double* __restrict__ y,
-                                 const double* __restrict__ z, size_t np, double sc, float4* __restrict__ pp,
-                                 uint32_t* __restrict__ ncount, int* __restrict__ cellroot, int* __restrict__ wcellroot,
-                                 size_t ncell, uint32_t* __restrict__ dsz, unsigned long long* __restrict__ counters) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (blockIdx.x == 0 && threadIdx.x < 64) tree_reset(threadIdx.x, dsz, counters);
-    if (i < np) {
-        if (pp) pp[i] = make_float4((float)(x[i] * sc), (float)(y[i] * sc), (float)(z[i] * sc), 1.0f);
-        ncount[i] = 0u;
-    }
-    if (i < ncell) {
-        cellroot[i] = -1;
-        if (wcellroot) wcellroot[i] = -1;
-    }
-}
-
 // node count on the device, clamped to the array capacity
 __device__ inline size_t dev_count(const uint32_t* __restrict__ dsz, int which, size_t cap) {
     size_t c = dsz[which];
@@ -258,166 +235,274 @@ __device__ inline size_t dev_count(const uint32_t* __restrict__ dsz, int which, 
 }
 
 // ---------------------------------------------------------------------------------------
-// Top-down build, one level per launch. A node record is (first particle, count, level, children)
-// in the order it was made; the records of level l are contiguous (dsz[DSZ_LOFF + l], count
-// dsz[DSZ_LVL + l]), which is also the level order the moments use. Cells of the chaining level L
-// are the roots; a node of more than nleaf particles above level 16 splits into its non-empty
-// octants, found by 8 lanes bisecting the node's key range in parallel, one octant boundary each.
-// Afterwards every node gets its pre-order index (first particle, then level): nodes that begin at
-// particle f are a chain of consecutive levels from lmin(f) = max(L, 1 + digits f shares with f-1),
-// so index = (nodes beginning before f) + level - lmin(f), with the first term from a scan of
-// per-particle node counts. The index does not depend on the order in which records were made,
-// so the numbering (and everything downstream) is deterministic.
+// Build from the sorted keys, all levels at once. Cells of the chaining level L are the roots; a
+// node of more than nleaf particles above the depth limit D splits into its non-empty octants. Which
+// nodes begin at particle f follows from the keys around it, whatever the other levels hold:
+//   - the first level at which f starts a prefix of its own is l1 = max(L, 1 + digits shared with
+//     f - 1); a node begins there if l1 = L, or if its parent, the prefix of l1 - 1 digits around f,
+//     holds more than nleaf particles (as many of its neighbours within nleaf places either way say);
+//   - below a node that begins at f, the next level's node begins at f too while f and f + nleaf share
+//     the level's digits (the node then holds more than nleaf).
+// So f's nodes are the levels l1 .. lk, and one pass over the particles counts them, a scan of the
+// counts per block of TB_PART particles places them, and a second pass writes them: three launches
+// where splitting level by level took two a level and a scan over the particles. Sort excluded, a
+// build with its moments and groups took 0.38 ms for 128^3 clustered particles, 0.20 for 32^3; now
+// 0.22 and 0.14.
+// Records are level by level and in particle order within a level, so the children of a node are
+// consecutive records; a node's own count (if it is no leaf) and number of children are filled in by
+// the moments, which visit them anyway. The order is the same from run to run.
+constexpr int TB_THREADS = 256;
+constexpr int TB_ITEMS = 4;
+constexpr int TB_PART = TB_THREADS * TB_ITEMS;  // particles per block
+constexpr int TB_LEAF_MAX = 256;                // largest nleaf (lagpm_box_set_tuning)
+constexpr int TB_ROWS = LAGPM_KEY_BITS + 3;     // counts per block: a row a level, all nodes, nodes beyond the limit
+constexpr int TB_SEQ = TB_PART / 64;            // runs of 64 particles of a block, in particle order
 
-// Append for the lanes whose flag is set: one atomic per wave, slots in lane order. Every lane of
-// the wave must call it.
-__device__ inline uint32_t wave_append(bool make, uint32_t* counter) {
-    const unsigned long long m = __ballot(make);
-    if (!m) return 0u;
-    const int leader = __ffsll((long long)m) - 1;
-    uint32_t base = 0u;
-    if ((int)(threadIdx.x & 63) == leader) base = atomicAdd(counter, (uint32_t)__popcll(m));
-    base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);
-    return base + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-}
-// the level-L cells that hold particles, one thread per cell (Morton index c = the key prefix)
-__global__ void cells_kernel(const uint64_t* __restrict__ K, size_t N, int L, size_t cap, uint32_t* __restrict__ dsz,
-                             int4* __restrict__ rec, uint32_t* __restrict__ ncount) {
-    const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t ncell = (size_t)1 << (3 * L);
-    uint32_t a = 0u, cnt = 0u;
-    if (c < ncell) {
-        const int sh = key_shift(L);
-        a = (uint32_t)lower_bound_pfx(K, 0, N, (uint64_t)c, sh);
-        cnt = (uint32_t)(upper_bound_pfx(K, a, N, (uint64_t)c, sh) - a);
+// the block's keys with nleaf neighbours either way: s[i] is the key of particle base - nleaf + i
+__device__ inline void tb_load_keys(const uint64_t* __restrict__ K, size_t N, long long base, int nleaf, uint64_t* s) {
+    for (int i = threadIdx.x; i < TB_PART + 2 * nleaf; i += TB_THREADS) {
+        const long long q = base - nleaf + i;
+        s[i] = q >= 0 && q < (long long)N ? K[q] : 0ull;
     }
-    const bool make = cnt > 0u;
-    const uint32_t r = wave_append(make, &dsz[DSZ_NODES]);
-    if (make) {
-        if (r < cap) {
-            rec[r] = make_int4((int)a, (int)cnt, L, 0);
-            ncount[a] += 1u;  // one node per first particle per level: no race
-        } else {
-            dsz[DSZ_OVERFLOW] = 1u;
+    __syncthreads();
+}
+// Levels l1 .. lk of the nodes that begin at particle f = base + i - nleaf (k = s + i, its key); lk <
+// l1: none. cf: digits that f shares with f + nleaf (-1 past the end).
+__device__ inline void tb_levels(const uint64_t* k, size_t f, size_t N, int nleaf, int L, int D, int& l1, int& lk, int& cf) {
+    const int b = f == 0 ? -1 : common_digits(k[-1], k[0]);
+    l1 = max(L, b + 1);
+    lk = l1 - 1;
+    cf = f + nleaf < N ? common_digits(k[0], k[nleaf]) : -1;
+    if (l1 > D) return;
+    if (l1 > L) {  // the parent (level b) holds f and f - 1: more than nleaf particles?
+        const int sh = key_shift(b);
+        const uint64_t pfx = k[0] >> sh;
+        int lo = f < (size_t)nleaf ? -(int)f : -nleaf, hi = -1;  // first place of the parent among the nleaf before f
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if ((k[mid] >> sh) == pfx) hi = mid;
+            else lo = mid + 1;
         }
+        int a = 0, e = N - 1 - f < (size_t)nleaf ? (int)(N - 1 - f) : nleaf;  // last one among the nleaf after f
+        while (a < e) {
+            const int mid = (a + e + 1) >> 1;
+            if ((k[mid] >> sh) == pfx) a = mid;
+            else e = mid - 1;
+        }
+        if (a - lo + 1 <= nleaf) return;
+    }
+    lk = min(max(l1, cf + 1), D);
+}
+
+// Pass 1: the block's nodes per level, their sum, and the nodes that should split beyond the limit;
+// beside it the cell roots cleared and (FP32 tree, pp non-null) the pp copy of the positions in units
+// of the particle mass.
+// pp is the FP32 copy of the positions for the tree, scaled by sc (rounded once from the FP64
+// product): with the log-r^2 force tables sc = sqrt(lam), so a pair's r^2 in these units is lam r^2,
+// the table variable, and needs no multiply in the pair loop. Everything the FP32 tree derives
+// from pp (centres, second moments, node sizes, group boxes) is in the same units.
+__global__ void __launch_bounds__(TB_THREADS) tree_count_kernel(const uint64_t* __restrict__ K, size_t N, int nleaf, int L, int D,
+                                                                const double* __restrict__ x, const double* __restrict__ y,
+                                                                const double* __restrict__ z, double sc, float4* __restrict__ pp,
+                                                                int* __restrict__ cellroot, size_t ncell,
+                                                                uint32_t* __restrict__ cnt, uint32_t nblk) {
+    __shared__ uint64_t s[TB_PART + 2 * TB_LEAF_MAX];
+    __shared__ uint32_t rows[TB_ROWS];
+    for (size_t c = (size_t)blockIdx.x * TB_THREADS + threadIdx.x; c < ncell; c += (size_t)gridDim.x * TB_THREADS) cellroot[c] = -1;
+    if (blockIdx.x >= nblk) return;
+    if (threadIdx.x < TB_ROWS) rows[threadIdx.x] = 0u;
+    const long long base = (long long)blockIdx.x * TB_PART;
+    tb_load_keys(K, N, base, nleaf, s);
+    const int lane = threadIdx.x & 63, nlev = D - L + 1;
+    uint32_t mine = 0u;  // lane j: row j's count over this wave's particles
+#pragma unroll
+    for (int q = 0; q < TB_ITEMS; q++) {
+        const int i = q * TB_THREADS + (int)threadIdx.x;
+        const size_t f = (size_t)base + i;
+        int l1 = 1, lk = 0, cf = -1;
+        if (f < N) {
+            tb_levels(s + nleaf + i, f, N, nleaf, L, D, l1, lk, cf);
+            if (pp) pp[f] = make_float4((float)(x[f] * sc), (float)(y[f] * sc), (float)(z[f] * sc), 1.0f);
+        }
+        uint32_t all = 0u;
+        for (int j = 0; j < nlev; j++) {
+            const uint32_t c = (uint32_t)__popcll(__ballot(l1 <= L + j && L + j <= lk));
+            all += c;
+            if (lane == j) mine += c;
+        }
+        if (lane == nlev) mine += all;
+        const uint32_t deep = (uint32_t)__popcll(__ballot(lk == D && cf >= D && D < LAGPM_KEY_BITS && l1 <= lk));
+        if (lane == nlev + 1) mine += deep;
+    }
+    if (lane < nlev + 2) atomicAdd(&rows[lane], mine);
+    __syncthreads();
+    if ((int)threadIdx.x < nlev + 2) cnt[(size_t)threadIdx.x * nblk + blockIdx.x] = rows[threadIdx.x];
+}
+// exclusive scan of one row of n counts by a workgroup of 256; the total is returned to all threads
+__device__ inline uint32_t block_row_scan(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, uint32_t n) {
+    __shared__ uint32_t wsum[4];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    uint32_t carry = 0u;
+    for (uint32_t c0 = 0; c0 < n; c0 += 2048) {
+        uint32_t v[8], t = 0u;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint32_t i = c0 + 8 * tid + k;
+            v[k] = i < n ? in[i] : 0u;
+            t += v[k];
+        }
+        int wt;
+        uint32_t run = (uint32_t)wave_excl_scan((int)t, lane, wt);
+        if (lane == 0) wsum[wid] = (uint32_t)wt;
+        __syncthreads();
+        uint32_t sum = 0u;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            if (w < wid) run += wsum[w];
+            sum += wsum[w];
+        }
+        run += carry;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint32_t i = c0 + 8 * tid + k;
+            if (i < n) out[i] = run;
+            run += v[k];
+        }
+        carry += sum;
+        __syncthreads();
+    }
+    return carry;
+}
+// One workgroup per row: its offsets per block, and what the rows' totals say (a level's nodes, all
+// nodes, whether the limit was met). The row of all nodes clears the other sizes and the counters.
+__global__ void __launch_bounds__(256) tree_rows_kernel(const uint32_t* __restrict__ cnt, uint32_t* __restrict__ off, uint32_t nblk,
+                                                        int L, int D, uint32_t* __restrict__ dsz,
+                                                        unsigned long long* __restrict__ counters) {
+    const int row = (int)blockIdx.x, nlev = D - L + 1;
+    const uint32_t total = block_row_scan(cnt + (size_t)row * nblk, off + (size_t)row * nblk, nblk);
+    const int t = (int)threadIdx.x;
+    if (row < nlev) {
+        if (t == 0) dsz[DSZ_LVL + L + row] = total;
+    } else if (row == nlev) {
+        if (t == 0) dsz[DSZ_NODES] = total;
+        if (t == DSZ_GROUPS || t == DSZ_WALKOVF || t == DSZ_TICKET) dsz[t] = 0u;
+        if (t <= LAGPM_KEY_BITS && (t < L || t > D)) dsz[DSZ_LVL + t] = 0u;
+        if (t < 4) counters[t] = 0ull;
+    } else if (t == 0) {
+        dsz[DSZ_DEEPER] = total ? 1u : 0u;
     }
 }
-// level l's records: from the previous level's end to the records made so far (clamped to cap)
-__global__ void level_mark_kernel(uint32_t* __restrict__ dsz, size_t cap, int l, int first_level) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const uint32_t made = dsz[DSZ_NODES] < cap ? dsz[DSZ_NODES] : (uint32_t)cap;
-    const uint32_t s = l == first_level ? 0u : dsz[DSZ_LOFF + l - 1] + dsz[DSZ_LVL + l - 1];
-    dsz[DSZ_LOFF + l] = s;
-    dsz[DSZ_LVL + l] = made - s;
-}
-// split the level-l records: 8 lanes per record, lane j finds where octant j begins. New
-// records are appended with one global atomic per workgroup and pass (a single counter that
-// every wave hit directly serialised ~10^5 atomics per level).
-constexpr int SPLIT_THREADS = 256;
-// At the depth limit (l == lmax) nothing is split: a record that would be is flagged instead.
-__global__ void __launch_bounds__(SPLIT_THREADS) split_kernel(const uint64_t* __restrict__ K, int l, int lmax, int nleaf,
-                                                              size_t cap, uint32_t* __restrict__ dsz, int4* __restrict__ rec,
-                                                              int* __restrict__ rch0, int* __restrict__ rch1,
-                                                              uint32_t* __restrict__ ncount, int* __restrict__ rfc) {
-    __shared__ uint32_t wcnt[SPLIT_THREADS / 64];
-    __shared__ uint32_t bbase;
-    const uint32_t n = dsz[DSZ_LVL + l], o = dsz[DSZ_LOFF + l];
-    const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int sub = (int)(threadIdx.x & 7), lane = (int)(threadIdx.x & 63), wid = (int)(threadIdx.x >> 6);
-    const size_t stride = (size_t)gridDim.x * blockDim.x / 8;
-    const size_t block_first = (size_t)blockIdx.x * blockDim.x / 8;
-    // every thread of the workgroup runs the same passes (the appends below are block-wide)
-    for (size_t pass = 0; block_first + pass < n; pass += stride) {
-        const size_t r = tid / 8 + pass;
-        const bool valid = r < n;
-        const int4 nd = valid ? rec[o + r] : make_int4(0, 0, 0, 0);
-        const bool need = valid && nd.y > nleaf && l < LAGPM_KEY_BITS;
-        if (need && l >= lmax) {
-            dsz[DSZ_DEEPER] = 1u;
-            dsz[DSZ_OVERFLOW] = 1u;  // the walk and the drift skip this box until it is redone
+// Pass 2: the records. link: first particle, count (leaves; the moments fill in the others), first
+// child record (0: a leaf; record 0 is a root), children (filled in); lev: level, and bit 8 for the
+// first child of its parent; rop: the record of each pre-order number (first particle, then level).
+__global__ void __launch_bounds__(TB_THREADS) tree_emit_kernel(const uint64_t* __restrict__ K, size_t N, int nleaf, int L, int D,
+                                                               const uint32_t* __restrict__ off, uint32_t nblk, size_t cap,
+                                                               uint32_t* __restrict__ dsz, int4* __restrict__ link,
+                                                               int* __restrict__ lev, uint32_t* __restrict__ rop,
+                                                               int* __restrict__ cellroot, int mcell) {
+    __shared__ uint64_t s[TB_PART + 2 * TB_LEAF_MAX];
+    __shared__ uint32_t wcnt[TB_SEQ][TB_ROWS];  // per run of 64 particles: its nodes per level, then the first record of each
+    const int nlev = D - L + 1, lane = (int)(threadIdx.x & 63), wid = (int)(threadIdx.x >> 6);
+    const bool over = dsz[DSZ_NODES] > cap || dsz[DSZ_DEEPER];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        uint32_t o = 0u;
+        for (int l = 0; l <= LAGPM_KEY_BITS; l++) {
+            dsz[DSZ_LOFF + l] = o;
+            o += dsz[DSZ_LVL + l];
         }
-        const bool split = need && l < lmax;
-        uint32_t b = 0u;
-        if (split) {
-            const uint64_t pfx = ((K[nd.x] >> key_shift(l)) << 3) | (uint64_t)sub;
-            b = (uint32_t)lower_bound_pfx(K, (size_t)nd.x, (size_t)nd.x + nd.y, pfx, key_shift(l + 1));
+        dsz[DSZ_OVERFLOW] = over ? 1u : 0u;  // the walk and the drift skip this box until it is redone
+    }
+    if (over) return;
+    const long long base = (long long)blockIdx.x * TB_PART;
+    tb_load_keys(K, N, base, nleaf, s);
+    int l1[TB_ITEMS], lk[TB_ITEMS], cf[TB_ITEMS];
+#pragma unroll
+    for (int q = 0; q < TB_ITEMS; q++) {
+        const int i = q * TB_THREADS + (int)threadIdx.x;
+        const size_t f = (size_t)base + i;
+        l1[q] = 1; lk[q] = 0; cf[q] = -1;
+        if (f < N) tb_levels(s + nleaf + i, f, N, nleaf, L, D, l1[q], lk[q], cf[q]);
+        uint32_t mine = 0u, all = 0u;
+        for (int j = 0; j < nlev; j++) {
+            const uint32_t c = (uint32_t)__popcll(__ballot(l1[q] <= L + j && L + j <= lk[q]));
+            all += c;
+            if (lane == j) mine = c;
         }
-        const uint32_t bn = (uint32_t)__shfl_down((int)b, 1, 64);
-        const uint32_t e = sub == 7 ? (uint32_t)(nd.x + nd.y) : bn;
-        const bool make = split && e > b;
-        const unsigned long long wm = __ballot(make);
-        if (lane == 0) wcnt[wid] = (uint32_t)__popcll(wm);
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            uint32_t t = 0;
-            for (int w = 0; w < SPLIT_THREADS / 64; w++) t += wcnt[w];
-            bbase = t ? atomicAdd(&dsz[DSZ_NODES], t) : 0u;
+        if (lane == nlev) mine = all;
+        if (lane <= nlev) wcnt[q * (TB_THREADS / 64) + wid][lane] = mine;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x <= nlev) {
+        const int j = (int)threadIdx.x;
+        uint32_t run = off[(size_t)j * nblk + blockIdx.x];
+        if (j < nlev)
+            for (int l = L; l < L + j; l++) run += dsz[DSZ_LVL + l];
+        for (int q = 0; q < TB_SEQ; q++) {
+            const uint32_t c = wcnt[q][j];
+            wcnt[q][j] = run;
+            run += c;
         }
-        __syncthreads();
-        uint32_t rr = bbase;
-        for (int w = 0; w < wid; w++) rr += wcnt[w];
-        rr += __builtin_amdgcn_mbcnt_hi((unsigned)(wm >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)wm, 0u));
-        __syncthreads();  // wcnt and bbase are rewritten by the next pass
-        if (make) {
-            if (rr < cap) {
-                rec[rr] = make_int4((int)b, (int)(e - b), l + 1, 0);
-                ncount[b] += 1u;
-            } else {
-                dsz[DSZ_OVERFLOW] = 1u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < TB_ITEMS; q++) {
+        const int i = q * TB_THREADS + (int)threadIdx.x, sq = q * (TB_THREADS / 64) + wid;
+        const size_t f = (size_t)base + i;
+        const uint64_t* k = s + nleaf + i;
+        auto below = [](unsigned long long m) {  // lanes below this one in m
+            return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+        };
+        uint32_t pre = wcnt[sq][nlev];
+        for (int j = 0; j < nlev; j++) pre += below(__ballot(l1[q] <= L + j && L + j <= lk[q]));
+        unsigned long long m = __ballot(l1[q] <= L && L <= lk[q]);
+        uint32_t r = wcnt[sq][0] + below(m);
+        for (int j = 0; j < nlev; j++) {
+            const int l = L + j;
+            const bool act = l1[q] <= l && l <= lk[q];
+            unsigned long long mn = 0ull;
+            uint32_t rn = 0u;
+            if (j + 1 < nlev) {
+                mn = __ballot(l1[q] <= l + 1 && l + 1 <= lk[q]);
+                rn = wcnt[sq][j + 1] + below(mn);
             }
+            if (act) {
+                uint32_t count = 0u;
+                const bool leaf = l == lk[q];
+                if (leaf) {
+                    const int sh = key_shift(l);
+                    const uint64_t pfx = k[0] >> sh;
+                    if (cf[q] < l) {  // ends within nleaf places
+                        int a = 0, e = N - 1 - f < (size_t)nleaf ? (int)(N - 1 - f) : nleaf;
+                        while (a < e) {
+                            const int mid = (a + e + 1) >> 1;
+                            if ((k[mid] >> sh) == pfx) a = mid;
+                            else e = mid - 1;
+                        }
+                        count = (uint32_t)(a + 1);
+                    } else {  // more than nleaf particles in one finest cell
+                        count = (uint32_t)(upper_bound_pfx(K, f + nleaf, N, pfx, sh) - f);
+                    }
+                }
+                link[r] = make_int4((int)f, (int)count, leaf ? 0 : (int)rn, 0);
+                lev[r] = l | (l > l1[q] ? 256 : 0);
+                rop[pre + (uint32_t)(l - l1[q])] = r;
+                if (l == L) {
+                    const uint64_t cell = k[0] >> key_shift(L);
+                    cellroot[compact3(cell) + (size_t)mcell * (compact3(cell >> 1) + (size_t)mcell * compact3(cell >> 2))] = (int)r;
+                }
+            }
+            m = mn;
+            r = rn;
         }
-        // the record's children, in octant order: lane j's rank among its group's non-empty octants
-        const unsigned long long mm = __ballot(make);
-        const uint32_t grp = (uint32_t)(mm >> (threadIdx.x & 56)) & 0xffu;
-        const int ci = __popc(grp & ((1u << sub) - 1u));
-        const size_t R = (size_t)o + r;
-        if (make) {
-            if (ci < 4) rch0[4 * R + ci] = (int)b;
-            else rch1[4 * R + ci - 4] = (int)b;
-            // the record's children are consecutive records (a record's lanes append in octant
-            // order, records in lane order): the first one's index is all the walk needs
-            if (ci == 0 && rfc) rfc[R] = (int)rr;
-        }
-        if (valid && sub == 0) rec[R].w = __popc(grp);
     }
 }
-__device__ inline int chain_first_level(const uint64_t* __restrict__ K, uint32_t f, int L) {
-    const int cpl = f == 0 ? -1 : common_digits(K[f - 1], K[f]);
-    return max(L, cpl + 1);
-}
-// pre-order numbering: info, child and parent links, cell roots and the level order
-__global__ void number_kernel(const uint64_t* __restrict__ K, int L, size_t cap, uint32_t* __restrict__ dsz,
-                              const int4* __restrict__ rec, const int* __restrict__ rch0, const int* __restrict__ rch1,
-                              const uint32_t* __restrict__ noff, int4* __restrict__ info, int* __restrict__ child,
-                              int* __restrict__ parent, int* __restrict__ cellroot, int mcell, uint32_t* __restrict__ order,
-                              const int* __restrict__ rfc, int4* __restrict__ wlink, int* __restrict__ wcellroot) {
-    const size_t r = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (dsz[DSZ_OVERFLOW] || r >= dev_count(dsz, DSZ_NODES, cap)) return;  // an overflowed build is redone
-    const int4 nd = rec[r];  // (first, count, level, children)
-    const uint32_t v = noff[nd.x] + (uint32_t)(nd.z - chain_first_level(K, (uint32_t)nd.x, L));
-    if ((size_t)v >= cap) return;  // cannot happen for sorted keys (the chain levels are consecutive)
-    order[r] = v;
-    info[v] = make_int4(nd.x, nd.y, nd.w, nd.z);
-    // the FP32 walk's links, by record: first particle, count, first child record, children
-    if (wlink) wlink[r] = make_int4(nd.x, nd.y, nd.w > 0 ? rfc[r] : 0, nd.w);
-    if (nd.z == L) {
-        parent[v] = -1;
-        const uint64_t cell = K[nd.x] >> key_shift(L);
-        const size_t ci = compact3(cell) + (size_t)mcell * (compact3(cell >> 1) + (size_t)mcell * compact3(cell >> 2));
-        cellroot[ci] = (int)v;
-        if (wcellroot) wcellroot[ci] = (int)r;
-    }
-    const uint32_t nodes = dsz[DSZ_NODES];
-    for (int c = 0; c < nd.w; c++) {
-        const uint32_t cf = (uint32_t)(c < 4 ? rch0[4 * r + c] : rch1[4 * r + c - 4]);
-        const uint32_t vc = noff[cf] + (uint32_t)(nd.z + 1 - chain_first_level(K, cf, L));
-        if (vc >= nodes) {  // cannot happen for sorted keys; the build is then marked failed
-            dsz[DSZ_OVERFLOW] = 1u;
-            return;
-        }
-        child[8 * (size_t)v + c] = (int)vc;
-        parent[vc] = (int)v;
-    }
+// A record's children: record fc and those after it up to the next first child (bit 8 of lev) or the
+// level's end. Every lane of the record's row of 8 calls it (sub: its index in the row).
+__device__ inline int row_children(const int* __restrict__ lev, int fc, int sub, uint32_t level_end) {
+    const uint32_t c = (uint32_t)fc + (uint32_t)sub;
+    const bool stop = fc == 0 || c >= level_end || (sub > 0 && (lev[c] & 256));
+    const uint32_t row = (uint32_t)(__ballot(stop) >> (threadIdx.x & 56)) & 0xffu;
+    return fc == 0 ? 0 : (row ? __ffs((int)row) - 1 : 8);
 }
 
 __device__ inline void kahan(float& s, float& c, float v) {
@@ -432,8 +517,9 @@ __device__ inline void kahan(float& s, float& c, float v) {
 // row's partial sums meet in a butterfly. Each lane sums with Kahan compensation, relative to the
 // node's first member (or first child's com); the compensated lane sums are then added in a fixed
 // order, so the moments are deterministic. Leaves read their particles; inner nodes read their
-// children's moments, which the previous level's launch wrote (and inner nodes of at most
-// RMAX_EXACT_MAX particles read their particles again for the exact rmax).
+// children's moments, consecutive records which the previous level's launch wrote, and get their
+// count and number of children on the way (and inner nodes of at most RMAX_EXACT_MAX particles read
+// their particles again for the exact rmax).
 constexpr int MOM_ROW = 8;  // lanes per node: a leaf's <= 32 particles are 4 per lane, an inner node's <= 8 children 1
 __device__ inline float row_sum(float v) {
 #pragma unroll
@@ -445,17 +531,22 @@ __device__ inline float row_max(float v) {
     for (int o = MOM_ROW / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, MOM_ROW));
     return v;
 }
-// every lane of the node's row calls this with its index `sub` in the row
-__device__ inline void moments_f32_node(size_t v, size_t rec, int sub, const float4* __restrict__ pp, const int4* __restrict__ info,
-                                        const int* __restrict__ child, float4* __restrict__ com, float4* __restrict__ q0,
-                                        float4* __restrict__ q1, float4* __restrict__ wgeo, float4* __restrict__ wq0,
-                                        float4* __restrict__ wq1) {
-    const int4 nd = info[v];
+__device__ inline int row_sum(int v) {
+#pragma unroll
+    for (int o = MOM_ROW / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, MOM_ROW);
+    return v;
+}
+// every lane of the record's row calls this with its index `sub` in the row
+__device__ inline void moments_f32_node(size_t r8, int sub, uint32_t level_end, const float4* __restrict__ pp,
+                                        const int* __restrict__ lev, int4* __restrict__ link, float4* __restrict__ geo,
+                                        float4* __restrict__ q0, float4* __restrict__ q1) {
+    int4 nd = link[r8];
+    const int nch = row_children(lev, nd.z, sub, level_end);
     float M = 0, cM = 0, Sx = 0, cx = 0, Sy = 0, cy = 0, Sz = 0, cz = 0;
     float Q[6] = {0, 0, 0, 0, 0, 0}, cQ[6] = {0, 0, 0, 0, 0, 0};
     float r2max = 0.f, rbound = 0.f;
     float3 cm;
-    if (nd.z == 0) {
+    if (nch == 0) {
         const float4 r = pp[nd.x];
         for (int p = nd.x + sub; p < nd.x + nd.y; p += MOM_ROW) {
             const float4 a = pp[p];
@@ -478,16 +569,25 @@ __device__ inline void moments_f32_node(size_t v, size_t rec, int sub, const flo
             r2max = fmaxf(r2max, dx * dx + dy * dy + dz * dz);
         }
     } else {
-        // lane c < nd.z takes child c
-        const bool has = sub < nd.z;
-        const int cv = has ? child[8 * v + sub] : 0;
-        const float4 r = com[child[8 * v]];
-        const float4 a = has ? com[cv] : make_float4(0.f, 0.f, 0.f, 0.f);
+        // lane c < nch takes child c
+        const bool has = sub < nch;
+        const size_t cv = (size_t)nd.z + (has ? sub : 0);
+        nd.y = row_sum(has ? link[cv].y : 0);
+        nd.w = nch;
+        const float4 r = geo[nd.z];
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b0 = a, b1 = a;
+        float rc = 0.f;
+        if (has) {
+            a = geo[cv];
+            b0 = q0[cv];
+            b1 = q1[cv];
+            rc = a.w;    // the child's rmax
+            a.w = b1.w;  // and mass
+        }
         M = row_sum(a.w);
         cm = make_float3(r.x + row_sum(a.w * (a.x - r.x)) / M, r.y + row_sum(a.w * (a.y - r.y)) / M,
                          r.z + row_sum(a.w * (a.z - r.z)) / M);
         if (has) {
-            const float4 b0 = q0[cv], b1 = q1[cv];
             const float dx = a.x - cm.x, dy = a.y - cm.y, dz = a.z - cm.z;
             Q[0] = b0.x + a.w * dx * dx;
             Q[1] = b0.y + a.w * dy * dy;
@@ -495,7 +595,7 @@ __device__ inline void moments_f32_node(size_t v, size_t rec, int sub, const flo
             Q[3] = b0.w + a.w * dx * dy;
             Q[4] = b1.x + a.w * dx * dz;
             Q[5] = b1.y + a.w * dy * dz;
-            rbound = sqrtf(dx * dx + dy * dy + dz * dz) + b1.w;
+            rbound = sqrtf(dx * dx + dy * dy + dz * dz) + rc;
         }
         rbound = row_max(rbound);
         if (nd.y <= RMAX_EXACT_MAX) {
@@ -510,85 +610,106 @@ __device__ inline void moments_f32_node(size_t v, size_t rec, int sub, const flo
     for (int k = 0; k < 6; k++) Q[k] = row_sum(Q[k] - cQ[k]);
     r2max = row_max(r2max);
     if (sub == 0) {
-        const float rmax = nd.z == 0 || nd.y <= RMAX_EXACT_MAX ? sqrtf(r2max) : rbound;
-        com[v] = make_float4(cm.x, cm.y, cm.z, M);
-        q0[v] = make_float4(Q[0], Q[1], Q[2], Q[3]);
-        q1[v] = make_float4(Q[4], Q[5], Q[0] + Q[1] + Q[2], rmax);
-        // the walk's copy at the node's record: what the opening test reads in one load, and the
-        // quadrupole with the mass in place of rmax and half the trace (the walk's table holds the
-        // trace term's line doubled)
-        wgeo[rec] = make_float4(cm.x, cm.y, cm.z, rmax);
-        wq0[rec] = make_float4(Q[0], Q[1], Q[2], Q[3]);
-        wq1[rec] = make_float4(Q[4], Q[5], 0.5f * (Q[0] + Q[1] + Q[2]), M);
+        const float rmax = nch == 0 || nd.y <= RMAX_EXACT_MAX ? sqrtf(r2max) : rbound;
+        // the opening test reads centre and size in one load; the quadrupole goes with the mass and half
+        // the trace (the walk's table holds the trace term's line doubled)
+        geo[r8] = make_float4(cm.x, cm.y, cm.z, rmax);
+        q0[r8] = make_float4(Q[0], Q[1], Q[2], Q[3]);
+        q1[r8] = make_float4(Q[4], Q[5], 0.5f * (Q[0] + Q[1] + Q[2]), M);
+        if (nch) link[r8] = nd;
     }
 }
 
 constexpr int LEVEL_BLOCKS = 2048;  // grid of the per-level launches (grid-stride over the level)
 __global__ void moments_f32_kernel(const float4* __restrict__ pp, const uint32_t* __restrict__ dsz, int level,
-                                   const uint32_t* __restrict__ order, const int4* __restrict__ info,
-                                   const int* __restrict__ child, float4* __restrict__ com, float4* __restrict__ q0,
-                                   float4* __restrict__ q1, float4* __restrict__ wgeo, float4* __restrict__ wq0,
-                                   float4* __restrict__ wq1) {
+                                   const int* __restrict__ lev, int4* __restrict__ link, float4* __restrict__ geo,
+                                   float4* __restrict__ q0, float4* __restrict__ q1) {
     if (dsz[DSZ_OVERFLOW]) return;
     const uint32_t n = dsz[DSZ_LVL + level], o = dsz[DSZ_LOFF + level];
+    const uint32_t end = level < LAGPM_KEY_BITS ? o + n + dsz[DSZ_LVL + level + 1] : o + n;
     const int sub = (int)(threadIdx.x & (MOM_ROW - 1));
-    // a node's lanes share i, so they are active or done together and their shuffles stay among them
+    // a record's lanes share i, so they are active or done together and their shuffles stay among them
     for (size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) / MOM_ROW; i < n;
          i += (size_t)gridDim.x * blockDim.x / MOM_ROW)
-        moments_f32_node(order[o + i], o + i, sub, pp, info, child, com, q0, q1, wgeo, wq0, wq1);
+        moments_f32_node(o + i, sub, end, pp, lev, link, geo, q0, q1);
 }
 
-// FP64 moments for the plain FP64 path (12 doubles per node).
-__device__ inline void moments_f64_node(size_t v, const double* __restrict__ x, const double* __restrict__ y,
-                                        const double* __restrict__ z, double mass, const int4* __restrict__ info,
-                                        const int* __restrict__ child, double* __restrict__ nd_d) {
-    const int4 nd = info[v];
-    double M = 0, Sx = 0, Sy = 0, Sz = 0, Q[6] = {0, 0, 0, 0, 0, 0}, rmax = 0;
-    double cxx, cyy, czz;
-    if (nd.z == 0) {
-        for (int p = nd.x; p < nd.x + nd.y; p++) { M += mass; Sx += mass * x[p]; Sy += mass * y[p]; Sz += mass * z[p]; }
-        cxx = Sx / M; cyy = Sy / M; czz = Sz / M;
-        for (int p = nd.x; p < nd.x + nd.y; p++) {
-            double dx = x[p] - cxx, dy = y[p] - cyy, dz = z[p] - czz;
-            Q[0] += mass * dx * dx; Q[1] += mass * dy * dy; Q[2] += mass * dz * dz;
-            Q[3] += mass * dx * dy; Q[4] += mass * dx * dz; Q[5] += mass * dy * dz;
-            rmax = fmax(rmax, sqrt(dx * dx + dy * dy + dz * dz));
+// FP64 moments for the FP64 path (12 doubles per record), the same way.
+__device__ inline double row_sum(double v) {
+#pragma unroll
+    for (int o = MOM_ROW / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, MOM_ROW);
+    return v;
+}
+__device__ inline double row_max(double v) {
+#pragma unroll
+    for (int o = MOM_ROW / 2; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, MOM_ROW));
+    return v;
+}
+__device__ inline void moments_f64_node(size_t r8, int sub, uint32_t level_end, const double* __restrict__ x,
+                                        const double* __restrict__ y, const double* __restrict__ z, const int* __restrict__ lev,
+                                        int4* __restrict__ link, double* __restrict__ nd_d) {
+    int4 nd = link[r8];
+    const int nch = row_children(lev, nd.z, sub, level_end);
+    double M, Q[6] = {0, 0, 0, 0, 0, 0}, rmax = 0, cx, cy, cz;
+    if (nch == 0) {
+        const double rx = x[nd.x], ry = y[nd.x], rz = z[nd.x];
+        double Sx = 0, Sy = 0, Sz = 0;
+        for (int p = nd.x + sub; p < nd.x + nd.y; p += MOM_ROW) { Sx += x[p] - rx; Sy += y[p] - ry; Sz += z[p] - rz; }
+        M = (double)nd.y;
+        cx = rx + row_sum(Sx) / M; cy = ry + row_sum(Sy) / M; cz = rz + row_sum(Sz) / M;
+        for (int p = nd.x + sub; p < nd.x + nd.y; p += MOM_ROW) {
+            const double dx = x[p] - cx, dy = y[p] - cy, dz = z[p] - cz;
+            Q[0] += dx * dx; Q[1] += dy * dy; Q[2] += dz * dz;
+            Q[3] += dx * dy; Q[4] += dx * dz; Q[5] += dy * dz;
+            rmax = fmax(rmax, dx * dx + dy * dy + dz * dz);
         }
+        rmax = sqrt(rmax);
     } else {
-        for (int c = 0; c < nd.z; c++) {
-            const double* a = nd_d + 12 * (size_t)child[8 * v + c];
-            M += a[3]; Sx += a[3] * a[0]; Sy += a[3] * a[1]; Sz += a[3] * a[2];
-        }
-        cxx = Sx / M; cyy = Sy / M; czz = Sz / M;
-        for (int c = 0; c < nd.z; c++) {
-            const double* a = nd_d + 12 * (size_t)child[8 * v + c];
-            double dx = a[0] - cxx, dy = a[1] - cyy, dz = a[2] - czz, m = a[3];
-            Q[0] += a[4] + m * dx * dx; Q[1] += a[5] + m * dy * dy; Q[2] += a[6] + m * dz * dz;
-            Q[3] += a[7] + m * dx * dy; Q[4] += a[8] + m * dx * dz; Q[5] += a[9] + m * dy * dz;
-            rmax = fmax(rmax, sqrt(dx * dx + dy * dy + dz * dz) + a[11]);
+        const bool has = sub < nch;
+        const size_t cv = (size_t)nd.z + (has ? sub : 0);
+        nd.y = row_sum(has ? link[cv].y : 0);
+        nd.w = nch;
+        const double *a = nd_d + 12 * cv, *r = nd_d + 12 * (size_t)nd.z;
+        const double m = has ? a[3] : 0.0, rx = r[0], ry = r[1], rz = r[2];
+        M = row_sum(m);
+        cx = rx + row_sum(m * (a[0] - rx)) / M; cy = ry + row_sum(m * (a[1] - ry)) / M; cz = rz + row_sum(m * (a[2] - rz)) / M;
+        if (has) {
+            const double dx = a[0] - cx, dy = a[1] - cy, dz = a[2] - cz;
+            Q[0] = a[4] + m * dx * dx; Q[1] = a[5] + m * dy * dy; Q[2] = a[6] + m * dz * dz;
+            Q[3] = a[7] + m * dx * dy; Q[4] = a[8] + m * dx * dz; Q[5] = a[9] + m * dy * dz;
+            rmax = sqrt(dx * dx + dy * dy + dz * dz) + a[11];
         }
         if (nd.y <= RMAX_EXACT_MAX) {
             double r2 = 0;
-            for (int p = nd.x; p < nd.x + nd.y; p++) {
-                const double dx = x[p] - cxx, dy = y[p] - cyy, dz = z[p] - czz;
+            for (int p = nd.x + sub; p < nd.x + nd.y; p += MOM_ROW) {
+                const double dx = x[p] - cx, dy = y[p] - cy, dz = z[p] - cz;
                 r2 = fmax(r2, dx * dx + dy * dy + dz * dz);
             }
             rmax = sqrt(r2);
         }
     }
-    double* o = nd_d + 12 * v;
-    o[0] = cxx; o[1] = cyy; o[2] = czz; o[3] = M;
-    for (int k = 0; k < 6; k++) o[4 + k] = Q[k];
-    o[10] = Q[0] + Q[1] + Q[2];
-    o[11] = rmax;
+#pragma unroll
+    for (int k = 0; k < 6; k++) Q[k] = row_sum(Q[k]);
+    rmax = row_max(rmax);
+    if (sub == 0) {
+        double* o = nd_d + 12 * r8;
+        o[0] = cx; o[1] = cy; o[2] = cz; o[3] = M;
+        for (int k = 0; k < 6; k++) o[4 + k] = Q[k];
+        o[10] = Q[0] + Q[1] + Q[2];
+        o[11] = rmax;
+        if (nch) link[r8] = nd;
+    }
 }
 __global__ void moments_f64_kernel(const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ z,
-                                   double mass, const uint32_t* __restrict__ dsz, int level, const uint32_t* __restrict__ order,
-                                   const int4* __restrict__ info, const int* __restrict__ child, double* __restrict__ nd_d) {
+                                   const uint32_t* __restrict__ dsz, int level, const int* __restrict__ lev,
+                                   int4* __restrict__ link, double* __restrict__ nd_d) {
     if (dsz[DSZ_OVERFLOW]) return;
     const uint32_t n = dsz[DSZ_LVL + level], o = dsz[DSZ_LOFF + level];
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        moments_f64_node(order[o + i], x, y, z, mass, info, child, nd_d);
+    const uint32_t end = level < LAGPM_KEY_BITS ? o + n + dsz[DSZ_LVL + level + 1] : o + n;
+    const int sub = (int)(threadIdx.x & (MOM_ROW - 1));
+    for (size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) / MOM_ROW; i < n;
+         i += (size_t)gridDim.x * blockDim.x / MOM_ROW)
+        moments_f64_node(o + i, sub, end, x, y, z, lev, link, nd_d);
 }
 
 // Target groups. A node of at most G particles whose parent holds more than G is a group, as is
@@ -605,12 +726,10 @@ __global__ void moments_f64_kernel(const double* __restrict__ x, const double* _
 // into runs of exactly G consecutive particles (a run may end inside a child), so the runs of a
 // parent fill their wavefronts but the last, and each still lies inside its parent.
 template <typename F>
-__device__ inline uint32_t group_pack(const int4& nd, int L, int G, int runs, const int4* __restrict__ info,
-                                      const int* __restrict__ child, const int* __restrict__ parent, size_t v,
-                                      F&& emit) {
+__device__ inline uint32_t group_pack(const int4& nd, int level, int L, int G, int runs, const int4* __restrict__ link, F&& emit) {
     const bool packed = runs == 2;
     if (runs == 1) {
-        if (nd.w != L) return 0u;
+        if (level != L) return 0u;
         const uint32_t c = (uint32_t)((nd.y + G - 1) / G);
         for (uint32_t t = 0; t < c; t++) {
             const int b = nd.x + (int)t * G;
@@ -619,13 +738,11 @@ __device__ inline uint32_t group_pack(const int4& nd, int L, int G, int runs, co
         return c;
     }
     if (nd.y <= G) {
-        // a small node below the cell level belongs to its parent's runs (a node the child table
-        // does not link, parent -1, is a group of its own)
-        if (nd.w != L && parent[v] >= 0) return 0u;
+        if (level != L) return 0u;  // a small node below the cell level belongs to its parent's runs
         emit(nd.x, nd.y);
         return 1u;
     }
-    if (nd.z == 0) {
+    if (nd.w == 0) {
         const uint32_t c = (uint32_t)((nd.y + G - 1) / G);
         for (uint32_t t = 0; t < c; t++) {
             const int b = nd.x + (int)t * G;
@@ -635,8 +752,8 @@ __device__ inline uint32_t group_pack(const int4& nd, int L, int G, int runs, co
     }
     uint32_t c = 0;
     int rb = 0, rn = 0;  // the open run: first particle, count
-    for (int k = 0; k < nd.z; k++) {
-        const int4 ci = info[child[8 * v + k]];
+    for (int k = 0; k < nd.w; k++) {
+        const int4 ci = link[nd.z + k];
         if (ci.y > G) {  // a big child owns its own groups and ends the run
             if (rn) { emit(rb, rn); c++; rn = 0; }
             continue;
@@ -654,34 +771,83 @@ __device__ inline uint32_t group_pack(const int4& nd, int L, int G, int runs, co
     if (rn) { emit(rb, rn); c++; }
     return c;
 }
-__global__ void group_count_kernel(const uint32_t* __restrict__ dsz, size_t cap, int L, int G, int runs,
-                                   const int4* __restrict__ info,
-                                   const int* __restrict__ child, const int* __restrict__ parent,
-                                   uint32_t* __restrict__ gcnt) {
-    size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= cap) return;
-    if (dsz[DSZ_OVERFLOW] || v >= dev_count(dsz, DSZ_NODES, cap)) {  // entries past the node count scan as zero
-        gcnt[v] = 0u;
+// Groups in the nodes' pre-order (so neighbouring groups are near in space): counts per block of
+// GB_NODES nodes, a scan of the blocks' counts, and the groups themselves. Blocks past the node count
+// leave at once.
+constexpr int GB_THREADS = 256;
+constexpr int GB_ITEMS = 4;
+constexpr int GB_NODES = GB_THREADS * GB_ITEMS;
+__global__ void __launch_bounds__(GB_THREADS) group_count_kernel(const uint32_t* __restrict__ dsz, size_t cap, int L, int G, int runs,
+                                                                 const int4* __restrict__ link, const int* __restrict__ lev,
+                                                                 const uint32_t* __restrict__ rop, uint32_t* __restrict__ gcnt) {
+    __shared__ uint32_t sum;
+    const size_t n = dsz[DSZ_OVERFLOW] ? 0 : dev_count(dsz, DSZ_NODES, cap), first = (size_t)blockIdx.x * GB_NODES;
+    if (first >= n) {
+        if (threadIdx.x == 0) gcnt[blockIdx.x] = 0u;
         return;
     }
-    gcnt[v] = group_pack(info[v], L, G, runs, info, child, parent, v, [](int, int) {});
-}
-__global__ void group_write_kernel(uint32_t* __restrict__ dsz, size_t cap, size_t gcap, int L, int G, int runs,
-                                   const int4* __restrict__ info, const int* __restrict__ child,
-                                   const int* __restrict__ parent, const uint32_t* __restrict__ gcnt,
-                                   const uint32_t* __restrict__ goff,
-                                   int2* __restrict__ groups) {
-    size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (dsz[DSZ_OVERFLOW] || v >= dev_count(dsz, DSZ_NODES, cap)) return;
-    uint32_t c = gcnt[v];
-    if (!c) return;
-    if ((size_t)goff[v] + c > gcap) {
-        dsz[DSZ_OVERFLOW] = 1u;
-        return;
+    if (threadIdx.x == 0) sum = 0u;
+    __syncthreads();
+    uint32_t c = 0u;
+#pragma unroll
+    for (int q = 0; q < GB_ITEMS; q++) {
+        const size_t v = first + (size_t)q * GB_THREADS + threadIdx.x;
+        if (v < n) {
+            const uint32_t r = rop[v];
+            c += group_pack(link[r], lev[r] & 255, L, G, runs, link, [](int, int) {});
+        }
     }
-    uint32_t g = goff[v];
-    group_pack(info[v], L, G, runs, info, child, parent, v, [&](int b, int m) { groups[g++] = make_int2(b, m); });
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) c += (uint32_t)__shfl_xor((int)c, o, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&sum, c);
+    __syncthreads();
+    if (threadIdx.x == 0) gcnt[blockIdx.x] = sum;
 }
+__global__ void __launch_bounds__(256) group_rows_kernel(const uint32_t* __restrict__ gcnt, uint32_t* __restrict__ goff, uint32_t nblk,
+                                                         size_t gcap, uint32_t* __restrict__ dsz) {
+    const uint32_t total = block_row_scan(gcnt, goff, nblk);
+    if (threadIdx.x == 0) {
+        dsz[DSZ_GROUPS] = total;
+        if (total > gcap) dsz[DSZ_OVERFLOW] = 1u;
+    }
+}
+__global__ void __launch_bounds__(GB_THREADS) group_write_kernel(const uint32_t* __restrict__ dsz, size_t cap, int L, int G, int runs,
+                                                                 const int4* __restrict__ link, const int* __restrict__ lev,
+                                                                 const uint32_t* __restrict__ rop, const uint32_t* __restrict__ goff,
+                                                                 int2* __restrict__ groups) {
+    __shared__ uint32_t wsum[GB_NODES / 64];
+    const size_t n = dsz[DSZ_OVERFLOW] ? 0 : dev_count(dsz, DSZ_NODES, cap), first = (size_t)blockIdx.x * GB_NODES;
+    if (first >= n) return;
+    const int lane = (int)(threadIdx.x & 63), wid = (int)(threadIdx.x >> 6);
+    int4 nd[GB_ITEMS];
+    int level[GB_ITEMS];
+    uint32_t at[GB_ITEMS];
+#pragma unroll
+    for (int q = 0; q < GB_ITEMS; q++) {
+        const size_t v = first + (size_t)q * GB_THREADS + threadIdx.x;
+        uint32_t c = 0u;
+        nd[q] = make_int4(0, 0, 0, 0);
+        if (v < n) {
+            const uint32_t r = rop[v];
+            nd[q] = link[r];
+            level[q] = lev[r] & 255;
+            c = group_pack(nd[q], level[q], L, G, runs, link, [](int, int) {});
+        }
+        int wt;
+        at[q] = (uint32_t)wave_excl_scan((int)c, lane, wt);
+        if (!c) nd[q].y = 0;
+        if (lane == 0) wsum[q * (GB_THREADS / 64) + wid] = (uint32_t)wt;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < GB_ITEMS; q++) {
+        if (!nd[q].y) continue;
+        uint32_t g = goff[blockIdx.x] + at[q];
+        for (int w = 0; w < q * (GB_THREADS / 64) + wid; w++) g += wsum[w];
+        group_pack(nd[q], level[q], L, G, runs, link, [&](int b, int m) { groups[g++] = make_int2(b, m); });
+    }
+}
+
 // start of a tree build: clear the size words and the interaction counters (a kernel, not a
 // memset, so the step can be captured in a graph)
 __global__ void tree_reset_kernel(uint32_t* __restrict__ dsz, unsigned long long* __restrict__ counters) {
@@ -1369,8 +1535,7 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
 // boxes, the heaviest group's own time for small ones.
 struct walk64_args {
     const double *x, *y, *z;
-    const int4* info;
-    const int* child;
+    const int4* link;  // first particle, count, first child record, children
     const double* nd;
     const int* cellroot;
     const uint64_t* key;
@@ -1607,18 +1772,18 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f64_kernel(walk64_args A) {
                     double hx, hy, hz;
                     shift_of(nb, hx, hy, hz);
                     const double* m = A.nd + 12 * (size_t)v;
-                    nd = A.info[v];
+                    nd = A.link[v];
                     const double rmax = m[11];
                     const double dmin2 = box_dist2(m[0] + hx, m[1] + hy, m[2] + hz);
                     const double rr = A.rcut + rmax;
                     if (dmin2 > rr * rr) kind = 0;
                     else if (nd.y >= A.naccept && dmin2 >= rmax * rmax * A.inv_theta2) kind = 1;
-                    else kind = nd.z == 0 ? 2 : 3;
+                    else kind = nd.w == 0 ? 2 : 3;
                 }
                 int tot;
-                const int nch = kind == 3 ? nd.z : 0;
+                const int nch = kind == 3 ? nd.w : 0;
                 const int off = wave_excl_scan(nch, lane, tot);
-                for (int c = 0; c < nch; c++) stack[sp + off + c] = (A.child[8 * (size_t)v + c] << 5) | nb;
+                for (int c = 0; c < nch; c++) stack[sp + off + c] = ((nd.z + c) << 5) | nb;
                 sp += tot;
                 wave_sync();
                 if (!split && (lane & (S - 1)) != part) kind = 0;  // another wave's
@@ -1734,6 +1899,13 @@ double lagpm_tree_scale(const lagpm_box* box) {
     return box->tab && box->tab->logr2 ? std::sqrt((double)box->tab->lam) : 1.0;
 }
 
+// scratch of a build: counts and offsets of the particle blocks' rows and of the node blocks' groups
+static size_t tree_part_blocks(size_t np) { return (np + TB_PART - 1) / TB_PART; }
+static size_t tree_group_blocks(size_t cap) { return (cap + GB_NODES - 1) / GB_NODES; }
+size_t lagpm_tree_tmp_bytes(size_t np, size_t cap) {
+    return 2 * (TB_ROWS * tree_part_blocks(np) + tree_group_blocks(cap)) * sizeof(uint32_t);
+}
+
 int lagpm_tree_alloc(lagpm_ctx* ctx, lagpm_box* box, size_t cap) {
     const bool f64 = box->p.precision == LAGPM_PREC_FP64;
     if (cap > (size_t)LAGPM_MAX_NODES) {
@@ -1743,25 +1915,18 @@ int lagpm_tree_alloc(lagpm_ctx* ctx, lagpm_box* box, size_t cap) {
     }
     lagpm_box_graphs_release(box);  // captured steps refer to the old arrays
     const size_t gcap = cap + box->np / 64 + 1;
-    RCHK(regrow(ctx, &box->nd_info, cap));
-    RCHK(regrow(ctx, &box->nd_parent, cap));
-    RCHK(regrow(ctx, &box->nd_child, 8 * cap));
-    RCHK(regrow(ctx, &box->gflag, cap));
-    RCHK(regrow(ctx, &box->goff, cap));
+    RCHK(regrow(ctx, &box->nd_link, cap));
+    RCHK(regrow(ctx, &box->nd_lev, cap));
+    RCHK(regrow(ctx, &box->nd_rop, cap));
     RCHK(regrow(ctx, &box->groups, gcap));
     if (f64) {
         RCHK(regrow(ctx, &box->nd_d, 12 * cap));
     } else {
-        RCHK(regrow(ctx, &box->nd_com, cap));
+        RCHK(regrow(ctx, &box->nd_geo, cap));
         RCHK(regrow(ctx, &box->nd_q0, cap));
         RCHK(regrow(ctx, &box->nd_q1, cap));
-        RCHK(regrow(ctx, &box->w_link, cap));
-        RCHK(regrow(ctx, &box->w_geo, cap));
-        RCHK(regrow(ctx, &box->w_q0, cap));
-        RCHK(regrow(ctx, &box->w_q1, cap));
-        RCHK(regrow(ctx, &box->w_rfc, cap));
     }
-    const size_t need = std::max(lagpm_scan_tmp_bytes(cap), std::max(lagpm_scan_tmp_bytes(box->np), lagpm_sort_tmp_bytes(box->np)));
+    const size_t need = std::max(lagpm_tree_tmp_bytes(box->np, cap), lagpm_sort_tmp_bytes(box->np));
     if (need > box->scan_tmp_bytes) {
         RCHK(regrow(ctx, (char**)&box->scan_tmp, need));
         box->scan_tmp_bytes = need;
@@ -1833,69 +1998,40 @@ int lagpm_tree_build(lagpm_ctx* ctx, lagpm_box* box) {
         return LAGPM_OK;
     }
     if (!box->sorted) RCHK(lagpm_sort_particles(ctx, box));
-    // sizes, counters, node counts and cell roots cleared; for the FP32 tree the pp copy in units
-    // of the particle mass (the walk multiplies by it with the kick)
     const size_t ncell = (size_t)box->mcell * box->mcell * box->mcell;
-    hipLaunchKernelGGL(tree_prep_kernel, dim3(blocks_for(std::max(np, ncell), 256)), dim3(256), 0, st, box->x, box->y,
-                       box->z, np, f64 ? 1.0 : lagpm_tree_scale(box), f64 ? (float4*)nullptr : box->pp, box->ncount,
-                       box->cellroot, f64 ? (int*)nullptr : box->w_cellroot, ncell, box->dsz, box->counters);
-    HIPCHK(ctx, hipGetLastError());
-    // top-down build: records of level-L cells, then one split per level, then the numbering.
-    // The records and child lists live in the moment arrays until the moments overwrite them.
-    int4* rec;
-    int *rch0, *rch1;
-    if (f64) {
-        rec = reinterpret_cast<int4*>(box->nd_d);
-        rch0 = reinterpret_cast<int*>(box->nd_d) + 4 * cap;
-        rch1 = reinterpret_cast<int*>(box->nd_d) + 8 * cap;
-    } else {
-        rec = reinterpret_cast<int4*>(box->nd_com);
-        rch0 = reinterpret_cast<int*>(box->nd_q0);
-        rch1 = reinterpret_cast<int*>(box->nd_q1);
-    }
-    uint32_t* order = box->goff;  // level order (goff is free until the group scan)
-    hipLaunchKernelGGL(cells_kernel, dim3(blocks_for(ncell, 256)), dim3(256), 0, st, box->key, np, L, cap, box->dsz, rec,
-                       box->ncount);
-    hipLaunchKernelGGL(level_mark_kernel, dim3(1), dim3(64), 0, st, box->dsz, cap, L, L);
-    HIPCHK(ctx, hipGetLastError());
-    const unsigned lblocks = (unsigned)std::min<size_t>(LEVEL_BLOCKS, blocks_for(cap, 256));
-    const unsigned mblocks = (unsigned)std::min<size_t>(2 * LEVEL_BLOCKS, blocks_for(cap * MOM_ROW, 256));
     const int D = std::min(LAGPM_KEY_BITS, std::max(L, box->depth));
-    int* rfc = f64 ? (int*)nullptr : box->w_rfc;
-    for (int l = L; l < D; l++) {
-        hipLaunchKernelGGL(split_kernel, dim3(lblocks), dim3(SPLIT_THREADS), 0, st, box->key, l, D, nleaf, cap, box->dsz,
-                           rec, rch0, rch1, box->ncount, rfc);
-        hipLaunchKernelGGL(level_mark_kernel, dim3(1), dim3(64), 0, st, box->dsz, cap, l + 1, L);
-        HIPCHK(ctx, hipGetLastError());
-    }
-    if (D < LAGPM_KEY_BITS) {  // the limit level: flag a record that still needs splitting
-        hipLaunchKernelGGL(split_kernel, dim3(lblocks), dim3(SPLIT_THREADS), 0, st, box->key, D, D, nleaf, cap, box->dsz,
-                           rec, rch0, rch1, box->ncount, rfc);
-        HIPCHK(ctx, hipGetLastError());
-    }
-    RCHK(lagpm_exclusive_scan_u32(ctx, st, box->scan_tmp, box->ncount, box->noff, np, box->dsz + DSZ_SCRATCH));
-    hipLaunchKernelGGL(number_kernel, dim3(blocks_for(cap, 256)), dim3(256), 0, st, box->key, L, cap, box->dsz, rec, rch0,
-                       rch1, box->noff, box->nd_info, box->nd_child, box->nd_parent, box->cellroot, box->mcell, order, rfc,
-                       f64 ? (int4*)nullptr : box->w_link, f64 ? (int*)nullptr : box->w_cellroot);
+    const uint32_t nblk = (uint32_t)tree_part_blocks(np), gblk = (uint32_t)tree_group_blocks(cap);
+    uint32_t* cnt = box->scan_tmp;
+    uint32_t* off = cnt + (size_t)TB_ROWS * nblk;
+    uint32_t* gcnt = off + (size_t)TB_ROWS * nblk;
+    uint32_t* goff = gcnt + gblk;
+    hipLaunchKernelGGL(tree_count_kernel, dim3(std::max(nblk, blocks_for(ncell, 4 * TB_THREADS))), dim3(TB_THREADS), 0, st, box->key,
+                       np, nleaf, L, D, box->x, box->y, box->z, f64 ? 1.0 : lagpm_tree_scale(box), f64 ? (float4*)nullptr : box->pp,
+                       box->cellroot, ncell, cnt, nblk);
     HIPCHK(ctx, hipGetLastError());
+    hipLaunchKernelGGL(tree_rows_kernel, dim3((unsigned)(D - L + 3)), dim3(256), 0, st, cnt, off, nblk, L, D, box->dsz, box->counters);
+    HIPCHK(ctx, hipGetLastError());
+    hipLaunchKernelGGL(tree_emit_kernel, dim3(nblk), dim3(TB_THREADS), 0, st, box->key, np, nleaf, L, D, off, nblk, cap, box->dsz,
+                       box->nd_link, box->nd_lev, box->nd_rop, box->cellroot, box->mcell);
+    HIPCHK(ctx, hipGetLastError());
+    const unsigned mblocks = (unsigned)std::min<size_t>(2 * LEVEL_BLOCKS, blocks_for(cap * MOM_ROW, 256));
     for (int l = D; l >= L; l--) {  // levels below D hold no records
         if (f64)
-            hipLaunchKernelGGL(moments_f64_kernel, dim3(lblocks), dim3(256), 0, st, box->x, box->y, box->z, 1.0, box->dsz, l,
-                               order, box->nd_info, box->nd_child, box->nd_d);
-        else  // (MOM_ROW lanes per node: a larger grid keeps as many nodes in flight)
-            hipLaunchKernelGGL(moments_f32_kernel, dim3(mblocks), dim3(256), 0, st, box->pp, box->dsz, l, order,
-                               box->nd_info, box->nd_child, box->nd_com, box->nd_q0, box->nd_q1, box->w_geo, box->w_q0,
-                               box->w_q1);
+            hipLaunchKernelGGL(moments_f64_kernel, dim3(mblocks), dim3(256), 0, st, box->x, box->y, box->z, box->dsz, l, box->nd_lev,
+                               box->nd_link, box->nd_d);
+        else
+            hipLaunchKernelGGL(moments_f32_kernel, dim3(mblocks), dim3(256), 0, st, box->pp, box->dsz, l, box->nd_lev, box->nd_link,
+                               box->nd_geo, box->nd_q0, box->nd_q1);
         HIPCHK(ctx, hipGetLastError());
     }
-
     const int runs = box->tune.runs;
-    hipLaunchKernelGGL(group_count_kernel, dim3(blocks_for(cap, 256)), dim3(256), 0, st, box->dsz, cap, L, G, runs,
-                       box->nd_info, box->nd_child, box->nd_parent, box->gflag);
+    hipLaunchKernelGGL(group_count_kernel, dim3(gblk), dim3(GB_THREADS), 0, st, box->dsz, cap, L, G, runs, box->nd_link, box->nd_lev,
+                       box->nd_rop, gcnt);
     HIPCHK(ctx, hipGetLastError());
-    RCHK(lagpm_exclusive_scan_u32(ctx, st, box->scan_tmp, box->gflag, box->goff, cap, box->dsz + DSZ_GROUPS));
-    hipLaunchKernelGGL(group_write_kernel, dim3(blocks_for(cap, 256)), dim3(256), 0, st, box->dsz, cap, gcap, L, G, runs,
-                       box->nd_info, box->nd_child, box->nd_parent, box->gflag, box->goff, box->groups);
+    hipLaunchKernelGGL(group_rows_kernel, dim3(1), dim3(256), 0, st, gcnt, goff, gblk, gcap, box->dsz);
+    HIPCHK(ctx, hipGetLastError());
+    hipLaunchKernelGGL(group_write_kernel, dim3(gblk), dim3(GB_THREADS), 0, st, box->dsz, cap, L, G, runs, box->nd_link, box->nd_lev,
+                       box->nd_rop, goff, box->groups);
     HIPCHK(ctx, hipGetLastError());
     box->tree_built = true;
     return LAGPM_OK;
@@ -1919,8 +2055,8 @@ int lagpm_tree_walk_f32(lagpm_ctx* ctx, lagpm_box* const* boxes, const double* f
             return lagpm_fail(ctx, LAGPM_E_INVAL, "boxes of one walk launch must share the FP32 force table");
         const double th = box->p.theta;
         walk_box& A = hb[(size_t)b];
-        A.pp = box->pp; A.link = box->w_link; A.geo = box->w_geo; A.q0 = box->w_q0;
-        A.q1 = box->w_q1; A.cellroot = box->w_cellroot; A.groups = box->groups; A.key = box->key;
+        A.pp = box->pp; A.link = box->nd_link; A.geo = box->nd_geo; A.q0 = box->nd_q0;
+        A.q1 = box->nd_q1; A.cellroot = box->cellroot; A.groups = box->groups; A.key = box->key;
         A.tvx = box->alt[0]; A.tvy = box->alt[1]; A.tvz = box->alt[2];  // free between sorts
         A.counters = box->counters; A.dsz = box->dsz;
         if (sample) {  // the sampled particles as groups of one (sizes: the sample's own words)
@@ -1963,7 +2099,7 @@ int lagpm_tree_walk_f64(lagpm_ctx* ctx, lagpm_box* box, double fact, const walk_
     if (box->np == 0) return LAGPM_OK;
     const double th = box->p.theta;
     walk64_args A;
-    A.x = box->x; A.y = box->y; A.z = box->z; A.info = box->nd_info; A.child = box->nd_child;
+    A.x = box->x; A.y = box->y; A.z = box->z; A.link = box->nd_link;
     A.nd = box->nd_d; A.cellroot = box->cellroot;
     A.key = box->key; A.cell_shift = 3 * (LAGPM_KEY_BITS - box->level_cell);
     A.tab = box->tab->tabd; A.nbins = box->tab->nbins; A.lam = box->tab->lam;
@@ -2137,7 +2273,19 @@ extern "C" int lagpm_tree_nodes_get(lagpm_ctx* ctx, lagpm_box* box, size_t cap, 
     const size_t nn = std::min<size_t>(d[DSZ_NODES], box->node_cap);
     *nnodes = nn;
     if (cap < nn) return lagpm_fail(ctx, LAGPM_E_INVAL, "the arrays hold fewer nodes than the tree has (see *nnodes)");
-    if (info) RCHK(lagpm_d2h(ctx, info, box->nd_info, nn * sizeof(int4), box->st));
+    // the records in the nodes' pre-order
+    std::vector<uint32_t> rop(nn);
+    RCHK(lagpm_d2h(ctx, rop.data(), box->nd_rop, nn * sizeof(uint32_t), box->st));
+    if (info) {
+        std::vector<int4> link(nn);
+        std::vector<int> lev(nn);
+        RCHK(lagpm_d2h(ctx, link.data(), box->nd_link, nn * sizeof(int4), box->st));
+        RCHK(lagpm_d2h(ctx, lev.data(), box->nd_lev, nn * sizeof(int), box->st));
+        for (size_t v = 0; v < nn; v++) {
+            const int4 a = link[rop[v]];
+            info[4 * v] = a.x; info[4 * v + 1] = a.y; info[4 * v + 2] = a.w; info[4 * v + 3] = lev[rop[v]] & 255;
+        }
+    }
     if (order) RCHK(lagpm_d2h(ctx, order, box->id, box->np * sizeof(uint32_t), box->st));
     if (!com && !quad) return LAGPM_OK;
     const double mass = box->p.mass;
@@ -2145,7 +2293,7 @@ extern "C" int lagpm_tree_nodes_get(lagpm_ctx* ctx, lagpm_box* box, size_t cap, 
         std::vector<double> t(12 * nn);
         RCHK(lagpm_d2h(ctx, t.data(), box->nd_d, t.size() * sizeof(double), box->st));
         for (size_t v = 0; v < nn; v++) {
-            const double* a = &t[12 * v];
+            const double* a = &t[12 * (size_t)rop[v]];
             if (com) { com[4 * v] = a[0]; com[4 * v + 1] = a[1]; com[4 * v + 2] = a[2]; com[4 * v + 3] = a[3] * mass; }
             if (quad) {
                 for (int k = 0; k < 7; k++) quad[8 * v + k] = a[4 + k] * mass;
@@ -2155,19 +2303,21 @@ extern "C" int lagpm_tree_nodes_get(lagpm_ctx* ctx, lagpm_box* box, size_t cap, 
         return LAGPM_OK;
     }
     std::vector<float4> c(nn), q0(nn), q1(nn);
-    RCHK(lagpm_d2h(ctx, c.data(), box->nd_com, nn * sizeof(float4), box->st));
+    RCHK(lagpm_d2h(ctx, c.data(), box->nd_geo, nn * sizeof(float4), box->st));
     RCHK(lagpm_d2h(ctx, q0.data(), box->nd_q0, nn * sizeof(float4), box->st));
     RCHK(lagpm_d2h(ctx, q1.data(), box->nd_q1, nn * sizeof(float4), box->st));
     const double s = lagpm_tree_scale(box), s2 = s * s;
     for (size_t v = 0; v < nn; v++) {
+        const size_t r = rop[v];
         if (com) {
-            com[4 * v] = c[v].x / s; com[4 * v + 1] = c[v].y / s; com[4 * v + 2] = c[v].z / s;
-            com[4 * v + 3] = c[v].w * mass;
+            com[4 * v] = c[r].x / s; com[4 * v + 1] = c[r].y / s; com[4 * v + 2] = c[r].z / s;
+            com[4 * v + 3] = q1[r].w * mass;
         }
         if (quad) {
-            const double q[8] = {q0[v].x, q0[v].y, q0[v].z, q0[v].w, q1[v].x, q1[v].y, q1[v].z, q1[v].w};
+            // (the record holds half the trace and the mass beside the quadrupole, rmax beside the centre)
+            const double q[7] = {q0[r].x, q0[r].y, q0[r].z, q0[r].w, q1[r].x, q1[r].y, 2.0 * q1[r].z};
             for (int k = 0; k < 7; k++) quad[8 * v + k] = q[k] * mass / s2;
-            quad[8 * v + 7] = q[7] / s;
+            quad[8 * v + 7] = c[r].w / s;
         }
     }
     return LAGPM_OK;
