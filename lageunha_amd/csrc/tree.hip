@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -959,8 +960,15 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
     __shared__ uint32_t s_ppidx[WALK_WAVES][PP_CAP];
     __shared__ int s_stack[WALK_WAVES][LSTACK > 0 ? LSTACK : 1];
     __shared__ int s_pcidx[WALK_WAVES][PC_CAP];
-    __shared__ float4 s_pp[WALK_WAVES][64];
-    __shared__ float4 s_pc[WALK_WAVES][3][64];
+    // Staged particles need three words (their masses are 1) and a node's third record three (its
+    // fourth is the mass, kept beside the centre). With the log tables the LDS pipe is the bound
+    // (90 % busy at 256^3) and 12-byte entries take fewer of its cycles than 16-byte ones: walk
+    // 12.95 -> 12.55 ms at 256^3, its last vector spills gone with them. The reference law is bound by its arithmetic: 3.76 -> 3.90 ms with them, so it
+    // keeps the aligned ones.
+    using psrc = std::conditional_t<LOGT, float3, float4>;
+    __shared__ psrc s_pp[WALK_WAVES][64];
+    __shared__ float4 s_pc[WALK_WAVES][2][64];
+    __shared__ psrc s_pc2[WALK_WAVES][64];
     __shared__ float4 s_shift[WALK_WAVES][27];  // the group's image shift of each neighbour cell
     __shared__ unsigned s_done;  // bit x: range x was found exhausted by a wave of this workgroup
     if (threadIdx.x == 0) s_done = 0u;
@@ -970,10 +978,10 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     uint32_t* ppidx = s_ppidx[wid];
     int* pcidx = s_pcidx[wid];
-    float4* cpp = s_pp[wid];
+    psrc* cpp = s_pp[wid];
     float4* cpc0 = s_pc[wid][0];
     float4* cpc1 = s_pc[wid][1];
-    float4* cpc2 = s_pc[wid][2];
+    psrc* cpc2 = s_pc2[wid];
     int* gstack = stacks + (size_t)(blockIdx.x * WALK_WAVES + wid) * STACK_MAX;
     int* lstack = s_stack[wid];
     // stack entry i: LDS below LSTACK (96% of pop rounds stay there), global memory above
@@ -1128,12 +1136,16 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
             sy = sh.y;
             sz = sh.z;
         };
-        // Source chunks are staged in LDS as float4 (x, y, z, m); entries past m are far-away
+        // Source chunks are staged in LDS; entries past m are far-away
         // dummies of zero mass, so every lane runs the same unrolled trip count and the cutoff
         // is a select (no branch, no exec-mask loop).
         // (8 box lengths away: sources lie within one box length of [0, n), and n >= 4 cutoffs)
         const float4 dummy = make_float4(8.f * A.box, 8.f * A.box, 8.f * A.box, 0.f);
-        auto load_pp = [&](int start, int m) -> float4 {
+        auto to_src = [](const float4& q) -> psrc {
+            if constexpr (LOGT) return make_float3(q.x, q.y, q.z);
+            else return q;
+        };
+        auto load_pp = [&](int start, int m) -> psrc {
             float4 s = dummy;
             if (lane < m) {
                 uint32_t e = ppidx[start + lane];
@@ -1142,14 +1154,14 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
                 s = gld4(A.pp, e >> 5);
                 s.x += sx; s.y += sy; s.z += sz;
             }
-            return s;
+            return to_src(s);
         };
         // Pair sums over one staged chunk. Lane (tgt, rep) takes the sources rep, rep + R, ...
         // (neighbouring lanes read neighbouring entries: no LDS bank conflicts). R is a template
         // value here, so the loads of one round are immediate offsets from one address. Sources
         // are taken four at a time: their LDS loads, then their table loads, are issued together
         // so one wave's LDS latency overlaps its own arithmetic.
-        auto pp_one = [&](float4 s) {
+        auto pp_one = [&](psrc s) {
 #pragma unroll
             for (int i = 0; i < M; i++) {
                 float dx = xt[i].x - s.x, dy = xt[i].y - s.y, dz = xt[i].z - s.z;
@@ -1167,11 +1179,11 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
             constexpr int RR = decltype(rc)::value;
             constexpr int iters = 64 / RR;
             constexpr int U = M == 1 ? 4 : 2;  // sources per round: U M pairs in flight
-            const float4* src = cpp + rep;
+            const psrc* src = cpp + rep;
             if constexpr (iters >= U) {
 #pragma unroll 2
                 for (int k = 0; k < iters; k += U) {
-                    float4 s[U];
+                    psrc s[U];
                     float dx[U][M], dy[U][M], dz[U][M], r2[U][M];
                     bool any = false;
 #pragma unroll
@@ -1224,7 +1236,7 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
         // there, and the reference law's select zeroes it); it is dropped before it costs a chunk
         // slot. The margin keeps every dropped pair clear of the float-rounded table edge.
         const float rc2_keep = A.rc2 * (1.0f + 1.0e-5f);
-        auto near_group = [&](float4 q) -> bool {
+        auto near_group = [&](psrc q) -> bool {
             const float ddx = fmaxf(fmaxf(lox - q.x, q.x - hix), 0.f);
             const float ddy = fmaxf(fmaxf(loy - q.y, q.y - hiy), 0.f);
             const float ddz = fmaxf(fmaxf(loz - q.z, q.z - hiz), 0.f);
@@ -1233,7 +1245,7 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
         int fill = 0;  // staged particles in cpp[0, fill), wave-uniform
         // append the kept particles of one 64-entry block to the chunk, computing the chunk when it
         // fills; survivors past its end start the next chunk
-        auto stage_pp = [&](float4 q, bool keep) {
+        auto stage_pp = [&](psrc q, bool keep) {
             int tot;
             const int off = wave_excl_count(keep, tot);
             const int room = 64 - fill;
@@ -1253,9 +1265,9 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
         // stage `nblock` consecutive blocks of the list from entry `start` (the last may be
         // partial: `mlast` entries); the next block's global loads overlap this block's chunk
         auto flush_pp = [&](int start, int nblock, int mlast) {
-            float4 nxt = load_pp(start, nblock == 1 ? mlast : 64);
+            psrc nxt = load_pp(start, nblock == 1 ? mlast : 64);
             for (int c = 0; c < nblock; c++) {
-                const float4 cur = nxt;
+                const psrc cur = nxt;
                 if (c + 1 < nblock) nxt = load_pp(start + 64 * (c + 1), c + 2 == nblock ? mlast : 64);
                 stage_pp(cur, near_group(cur));  // entries past m are far dummies: never kept
             }
@@ -1263,7 +1275,7 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
         // One node interaction: monopole plus quadrupole, Q d computed once and reused for
         // d.Q.d (the quadratic form) and for the 2 f2 Q d term. The table's f2 line is stored
         // doubled and the node's trace halved (both exact), so 2 f2 is the table value itself.
-        auto pc_eval = [&](float4 c, float4 qa, float4 qb, float2 t0, float4 t12, float t, float dx, float dy, float dz,
+        auto pc_eval = [&](float4 c, float4 qa, psrc qb, float2 t0, float4 t12, float t, float dx, float dy, float dz,
                            bool in, float& ax, float& ay, float& az) {
             float f1 = t0.x + t0.y * t, f2 = t12.x + t12.y * t, f3 = t12.z + t12.w * t;
             float qx1 = qa.x * dx + qa.w * dy + qb.x * dz;
@@ -1281,7 +1293,7 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
             az = fmaf(qx3, two, fmaf(dz, tmp, az));
         };
         // one node against this lane's M targets
-        auto pc_node = [&](const float4& c, const float4& qa, const float4& qb) {
+        auto pc_node = [&](const float4& c, const float4& qa, const psrc& qb) {
 #pragma unroll
             for (int i = 0; i < M; i++) {
                 const float dx = xt[i].x - c.x, dy = xt[i].y - c.y, dz = xt[i].z - c.z;
@@ -1297,12 +1309,13 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
             constexpr int U = M == 1 ? 2 : 1;  // nodes per round: U M interactions in flight
             const float4* n0 = cpc0 + rep;
             const float4* n1 = cpc1 + rep;
-            const float4* n2 = cpc2 + rep;
+            const psrc* n2 = cpc2 + rep;
             if constexpr (iters >= 2) {
                 // the nodes' loads first, then their table loads, as for the particles
 #pragma unroll 2
                 for (int k = 0; k < iters; k += U) {
-                    float4 c[U], qa[U], qb[U];
+                    float4 c[U], qa[U];
+                    psrc qb[U];
                     float dx[U][M], dy[U][M], dz[U][M], r2[U][M];
                     bool any = false;
 #pragma unroll
@@ -1351,11 +1364,11 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
                 const float4 c = gld4(A.geo, v), q1 = gld4(A.q1, v);
                 cpc0[lane] = make_float4(c.x + sx, c.y + sy, c.z + sz, q1.w);  // (centre, mass)
                 cpc1[lane] = gld4(A.q0, v);
-                cpc2[lane] = q1;
+                cpc2[lane] = to_src(q1);
             } else {
                 cpc0[lane] = dummy;
                 cpc1[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-                cpc2[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+                cpc2[lane] = to_src(make_float4(0.f, 0.f, 0.f, 0.f));
             }
             wave_sync();
             if (R == 1) pc_chunk_r(ic<1>{});
@@ -1476,7 +1489,7 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
         if (pc_n > 0) flush_pc(0, pc_n);
         if (pp_n > 0) flush_pp(0, 1, pp_n);
         if (fill > 0) {  // the last, partial chunk: far zero-mass dummies after the staged particles
-            if (lane >= fill) cpp[lane] = dummy;
+            if (lane >= fill) cpp[lane] = to_src(dummy);
             wave_sync();
             pp_chunk();
             npp += (unsigned long long)fill;
