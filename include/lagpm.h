@@ -169,7 +169,7 @@ int lagpm_box_download_eunha(lagpm_ctx* ctx, lagpm_box* box, void* dm_bp, size_t
  * lies inside [fof_link, 4 - fof_link) on every axis with fewer than minnum members (the
  * reference fixes FOF_MINNUM = 20, PreFoF.c:273). flags (np bytes, caller order, may be NULL)
  * gets 1 for the particles of kept groups (the reference's FoFflag); nflagged their count.
- * Uses box->np * ~93 bytes of device scratch for the call. */
+ * Its scratch is the box's own; a box with few particles for its n takes n^3/16 bytes more for the call. */
 int lagpm_prefof(lagpm_ctx* ctx, lagpm_box* box, float fof_link, int minnum, uint8_t* flags, size_t* nflagged);
 
 /* ---- GOTPM particle files and records (host only, no GPU needed) --------------------- */
