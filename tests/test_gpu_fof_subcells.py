@@ -47,3 +47,18 @@ def test_a_particle_without_position_is_linked_to_none(ctx):
     rest = np.isfinite(bad).all(axis=1)
     want, _ = orc.prefof(16, bad[rest], 0.2, 35)
     assert np.array_equal(got[rest], want) and cnt == int(got.sum())
+
+
+@pytest.mark.parametrize("n,np_", [(128, 1), (128, 12), (64, 700)])
+def test_few_particles_in_a_large_box_and_the_box_afterwards(ctx, n, np_):
+    """The table of cells is larger than the box's own scratch; the box's particles are as they were."""
+    g = np.random.default_rng(np_)
+    pos = (8.0 + 0.3 * g.random((np_, 3))) % n
+    vel = g.normal(size=(np_, 3))
+    want, wcnt = orc.prefof(n, pos, 0.2, 5)
+    with lagpm.Box(ctx, lagpm.make_params(n), np_) as b:
+        b.upload_pos(pos, vel)
+        got, cnt = b.prefof(0.2, 5)
+        pos2, vel2 = b.download()
+    assert cnt == wcnt and np.array_equal(got, want)
+    assert np.array_equal(pos2, pos) and np.array_equal(vel2, vel)
