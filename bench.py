@@ -309,7 +309,7 @@ def ensemble(args, ctx, lagpm, ics):
            "sizes": sorted(n for n, _ in specs), "identical_plain_vs_batched": bool(same),
            "tree_tuning": {str(n): {"nleaf": t[0], "group": t[1], "group_mode": MODE_NAMES[t[2]]}
                            for n, t in sorted(tuned.items())},
-           "batch_pipeline": {"stages": 5, "reserve_cu": 32, "share_growth": 1.5,
+           "batch_pipeline": {"stages": min(5, (len(specs) + 2) // 4), "reserve_cu": 32, "share_growth": 1.5,
                               "note": "library default (lagpm_set_batch_pipeline)"}}
     for k in ("plain", "batched"):
         L = np.array(lat[k]) * 1e3

@@ -1252,10 +1252,15 @@ int batch_step(lagpm_ctx* ctx, lagpm_box* const* boxes, int nbox, const double* 
     // (one fused launch, leaving ctx->stage_reserve_cu CUs free) runs while the fronts of group
     // g+1 are on the pool streams, whose small kernels are latency bound and fill those CUs. Every
     // drift is queued after all fronts, so no front waits behind a walk on its pool stream.
-    int stages = std::max(1, ctx->batch_stages);
+    // Where the caller has not set the stages: up to five, about four boxes per group. A group's
+    // walk ends with its heaviest target groups, which many boxes hide and few do not. ms per step at
+    // 1 / 2 / 3 / 4 / 5 stages: 8 boxes of 32^3-96^3 4.36 4.68 4.91 5.19 5.24; 10 of them 5.78 5.39 5.05
+    // 5.29 5.55; 16 of them 7.76 8.13 7.79 7.87 7.85; 20 of them 10.3 9.58 9.62 9.37 9.43; 14 of
+    // 32^3-64^3 4.93 4.89 4.35 4.58 4.86; 30 of 32^3-64^3 8.75 8.64 8.44 8.25 8.01.
+    int stages = ctx->batch_stages ? std::min<int>(ctx->batch_stages, (int)(live.size() / 2))
+                                   : std::min<int>(5, (int)((live.size() + 2) / 4));
     for (lagpm_box* b : live)
         if (b->p.precision != LAGPM_PREC_FP32 || b->tab != live[0]->tab) stages = 1;
-    stages = std::min<int>(stages, (int)(live.size() / 2));  // at least two boxes per group
     if (stages < 2) stages = 1;
     int rc = LAGPM_OK;
     if (stages > 1) {

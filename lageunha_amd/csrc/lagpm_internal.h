@@ -75,7 +75,7 @@ struct lagpm_ctx {
     bool use_graphs = false;                 // capture box step fronts in hipGraphs (lagpm_set_step_graphs)
     bool step_events = false;                // record the phase events of step fronts (lagpm_set_step_graphs(ctx, 0))
     bool walk_census = false;                // FP32 walks count the pairs within the cutoff
-    int batch_stages = 5;                    // groups of a pipelined batch step (1: no pipeline)
+    int batch_stages = 0;                    // groups of a pipelined batch step (1: no pipeline; 0: by the boxes)
     int stage_reserve_cu = 32;               // CUs a non-final group's walk leaves to the next fronts
     hipEvent_t ev[4] = {};
     double* pk_scratch = nullptr;  // this device's static power-spectrum scratch (device address)
