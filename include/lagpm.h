@@ -100,7 +100,7 @@ typedef struct lagpm_tree_stats {
     double   ms_build;  /* sort + build + moments, device time */
     double   ms_walk;   /* walk kernel, device time */
     int32_t  deepest;   /* deepest tree level with nodes (levels of the 16-bit-per-axis keys) */
-    int32_t  depth_limit; /* deepest level the next build splits to (a deeper tree is detected
+    int32_t  depth_limit; /* deepest level the next tree is expected to use (a deeper one is detected
                              and rebuilt at full depth) */
     uint64_t n_pp_within; /* of n_pp, the pairs within the cutoff (FP32 walk with the census on,
                              lagpm_set_walk_census; 0 otherwise) */

@@ -128,10 +128,10 @@ struct lagpm_box {
     bool sorted = false;
     bool tree_built = false;  // a tree build has been queued (node arrays hold a tree)
     tree_tune tune;
-    // deepest level the build splits to: the full key depth until one build has run, then two
-    // levels below the deepest level that build used; a build that meets a node still to split
-    // at this limit flags it, and the tree is redone at full depth (levels below the tree's
-    // depth cost one empty launch each per kernel)
+    // deepest level the tree is expected to use: the full key depth until one build has run, then two
+    // levels below the deepest level that build used. It sets the key bits that the sort orders; a
+    // build that meets a node still to split where those end flags it, and the tree is redone at
+    // full depth
     int depth = LAGPM_KEY_BITS;
     hipStream_t st = nullptr;  // stream this box's work is queued on (context stream or a pool stream)
     hipStream_t st2 = nullptr;  // second stream of a step front (the tree build beside the PM kick)

@@ -634,6 +634,27 @@ __global__ void moments_f32_kernel(const float4* __restrict__ pp, const uint32_t
          i += (size_t)gridDim.x * blockDim.x / MOM_ROW)
         moments_f32_node(o + i, sub, end, pp, lev, link, geo, q0, q1);
 }
+// Levels `bottom` up to `top` in one launch of one workgroup, a barrier between levels: those below the
+// expected depth, mostly without a record.
+constexpr int MOM_DEEP_THREADS = 1024;
+template <typename F>
+__device__ inline void moments_deep(const uint32_t* __restrict__ dsz, int bottom, int top, F&& node) {
+    if (dsz[DSZ_OVERFLOW]) return;
+    for (int l = bottom; l >= top; l--) {
+        const uint32_t n = dsz[DSZ_LVL + l], o = dsz[DSZ_LOFF + l];
+        if (n == 0) continue;  // the same for every thread
+        const uint32_t end = l < LAGPM_KEY_BITS ? o + n + dsz[DSZ_LVL + l + 1] : o + n;
+        for (uint32_t i = threadIdx.x / MOM_ROW; i < n; i += MOM_DEEP_THREADS / MOM_ROW)
+            node((size_t)(o + i), (int)(threadIdx.x & (MOM_ROW - 1)), end);
+        __syncthreads();
+    }
+}
+__global__ void __launch_bounds__(MOM_DEEP_THREADS) moments_f32_deep_kernel(const float4* __restrict__ pp, const uint32_t* __restrict__ dsz,
+                                                                            int bottom, int top, const int* __restrict__ lev,
+                                                                            int4* link, float4* geo, float4* q0, float4* q1) {
+    moments_deep(dsz, bottom, top,
+                 [&](size_t r, int sub, uint32_t end) { moments_f32_node(r, sub, end, pp, lev, link, geo, q0, q1); });
+}
 
 // FP64 moments for the FP64 path (12 doubles per record), the same way.
 __device__ inline double row_sum(double v) {
@@ -711,6 +732,13 @@ __global__ void moments_f64_kernel(const double* __restrict__ x, const double* _
     for (size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) / MOM_ROW; i < n;
          i += (size_t)gridDim.x * blockDim.x / MOM_ROW)
         moments_f64_node(o + i, sub, end, x, y, z, lev, link, nd_d);
+}
+
+__global__ void __launch_bounds__(MOM_DEEP_THREADS) moments_f64_deep_kernel(const double* __restrict__ x, const double* __restrict__ y,
+                                                                            const double* __restrict__ z, const uint32_t* __restrict__ dsz,
+                                                                            int bottom, int top, const int* __restrict__ lev, int4* link,
+                                                                            double* nd_d) {
+    moments_deep(dsz, bottom, top, [&](size_t r, int sub, uint32_t end) { moments_f64_node(r, sub, end, x, y, z, lev, link, nd_d); });
 }
 
 // Target groups. A node of at most G particles whose parent holds more than G is a group, as is
@@ -1949,6 +1977,25 @@ int lagpm_tree_alloc(lagpm_ctx* ctx, lagpm_box* box, size_t cap) {
     return LAGPM_OK;
 }
 
+// The tree is expected to end above box->depth, so only the top 3 * depth key bits must be in order:
+// a box whose tree is shallower needs fewer passes. Below them the order is the previous one (the
+// sort is stable). An even number of passes leaves the result in key/perm, where captured steps and
+// the walk's descriptors expect it.
+static int sort_passes(const lagpm_box* box) {
+    const int D = std::min(LAGPM_KEY_BITS, std::max(box->level_cell, box->depth));
+    return (((3 * D + 7) / 8) + 1) & ~1;
+}
+// Levels a build may split to: down to box->depth, and a tree that needs more is detected and
+// redone after a full sort; but where the passes have put all key bits in order (depth 11 and more)
+// the build goes on below the limit itself, and gives what the redone one would. A halo that
+// tightens costs no second sort, build and walk then: a batch of 10 boxes (32^3-96^3) redid 9 trees in
+// 10 steps and took 5 of its 53 ms over them. The levels below the limit take their moments in one
+// launch: a launch each cost a 64^3 step 0.02 of 1.01 ms.
+static int build_depth(const lagpm_box* box) {
+    if (8 * sort_passes(box) >= 3 * LAGPM_KEY_BITS) return LAGPM_KEY_BITS;
+    return std::min(LAGPM_KEY_BITS, std::max(box->level_cell, box->depth));
+}
+
 int lagpm_sort_particles(lagpm_ctx* ctx, lagpm_box* box, const double* drag, hipStream_t vst) {
     const size_t np = box->np;
     if (np == 0) return LAGPM_OK;
@@ -1957,13 +2004,7 @@ int lagpm_sort_particles(lagpm_ctx* ctx, lagpm_box* box, const double* drag, hip
     hipLaunchKernelGGL(keys_kernel, dim3(blocks_for(np, 256)), dim3(256), 0, st, box->x, box->y, box->z, np, s,
                        box->key, box->perm);
     HIPCHK(ctx, hipGetLastError());
-    // The tree splits nodes down to box->depth at most (deeper trees are detected and redone after
-    // a full sort), so only the top 3 * depth key bits must be in order: a box whose tree is
-    // shallower needs fewer passes. Below them the order is the previous one (the sort is stable).
-    // An even number of passes leaves the result in key/perm, where captured steps and the walk's
-    // descriptors expect it.
-    const int D = std::min(LAGPM_KEY_BITS, std::max(box->level_cell, box->depth));
-    const int passes = (((3 * D + 7) / 8) + 1) & ~1;
+    const int passes = sort_passes(box);
     bool alt = false;
     RCHK(lagpm_radix_sort_pairs(ctx, st, box->scan_tmp, box->key, box->key2, box->perm, box->perm2, np, 8 * passes, &alt,
                                 3 * LAGPM_KEY_BITS - 8 * passes));
@@ -2012,7 +2053,7 @@ int lagpm_tree_build(lagpm_ctx* ctx, lagpm_box* box) {
     }
     if (!box->sorted) RCHK(lagpm_sort_particles(ctx, box));
     const size_t ncell = (size_t)box->mcell * box->mcell * box->mcell;
-    const int D = std::min(LAGPM_KEY_BITS, std::max(L, box->depth));
+    const int D = build_depth(box);
     const uint32_t nblk = (uint32_t)tree_part_blocks(np), gblk = (uint32_t)tree_group_blocks(cap);
     uint32_t* cnt = box->scan_tmp;
     uint32_t* off = cnt + (size_t)TB_ROWS * nblk;
@@ -2028,7 +2069,17 @@ int lagpm_tree_build(lagpm_ctx* ctx, lagpm_box* box) {
                        box->nd_link, box->nd_lev, box->nd_rop, box->cellroot, box->mcell);
     HIPCHK(ctx, hipGetLastError());
     const unsigned mblocks = (unsigned)std::min<size_t>(2 * LEVEL_BLOCKS, blocks_for(cap * MOM_ROW, 256));
-    for (int l = D; l >= L; l--) {  // levels below D hold no records
+    const int expected = std::min(D, std::max(L, box->depth));
+    if (expected < D) {
+        if (f64)
+            hipLaunchKernelGGL(moments_f64_deep_kernel, dim3(1), dim3(MOM_DEEP_THREADS), 0, st, box->x, box->y, box->z, box->dsz, D,
+                               expected + 1, box->nd_lev, box->nd_link, box->nd_d);
+        else
+            hipLaunchKernelGGL(moments_f32_deep_kernel, dim3(1), dim3(MOM_DEEP_THREADS), 0, st, box->pp, box->dsz, D, expected + 1,
+                               box->nd_lev, box->nd_link, box->nd_geo, box->nd_q0, box->nd_q1);
+        HIPCHK(ctx, hipGetLastError());
+    }
+    for (int l = expected; l >= L; l--) {  // levels below D hold no records
         if (f64)
             hipLaunchKernelGGL(moments_f64_kernel, dim3(mblocks), dim3(256), 0, st, box->x, box->y, box->z, box->dsz, l, box->nd_lev,
                                box->nd_link, box->nd_d);
@@ -2190,6 +2241,8 @@ int lagpm_tree_finish_with(lagpm_ctx* ctx, lagpm_box* box, const tree_readback& 
             box->depth = lim;
             lagpm_box_graphs_release(box);  // captured steps hold the old limit
         }
+    } else if (deepest > box->depth) {  // a build below the limit (build_depth): as a rebuild would set it
+        box->depth = std::min(LAGPM_KEY_BITS, deepest + 2);
     }
     if (c[2]) return lagpm_fail(ctx, LAGPM_E_OVERFLOW, "tree walk stack overflow in " + std::to_string(c[2]) + " groups");
     return LAGPM_OK;
