@@ -1208,7 +1208,66 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
             constexpr int iters = 64 / RR;
             constexpr int U = M == 1 ? 4 : 2;  // sources per round: U M pairs in flight
             const psrc* src = cpp + rep;
-            if constexpr (iters >= U) {
+            if constexpr (LOGT && M == 1 && iters >= 2 * U) {
+                // Two rounds in flight: while a round's table lines and the sources after it are on their
+                // way, the round before is added up. Where a walk lasts as long as its heaviest group, a wave
+                // by itself on its SIMD waits for every LDS read otherwise: 41 ns a source, of which 20
+                // are the issue of its operations. Walk 32^3 theta 0 0.61 -> 0.56 ms, 64^3
+                // 0.59 -> 0.56, 32^3 0.306 -> 0.293; with 16 waves a CU (256^3) 12.9 either way. Eight
+                // sources a round spill (256^3 28 ms), two gain nothing, three targets a lane neither (their
+                // rounds have six pairs). The fused operations are written out: the same bits as the plain loop.
+                constexpr int NB = iters / U;  // rounds, an even number
+                struct round {
+                    float dx[U], dy[U], dz[U], r2[U];
+                    float2 tb[U];
+                } P, Q;
+                psrc s[U];
+                auto load = [&](int b) {
+#pragma unroll
+                    for (int u = 0; u < U; u++) s[u] = src[(b * U + u) * RR];
+                };
+                auto diff = [&](round& B) {
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        B.dx[u] = xt[0].x - s[u].x; B.dy[u] = xt[0].y - s[u].y; B.dz[u] = xt[0].z - s[u].z;
+                    }
+                };
+                auto look = [&](round& B) {
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        B.r2[u] = fmaf(B.dz[u], B.dz[u], fmaf(B.dx[u], B.dx[u], B.dy[u] * B.dy[u]));
+                        if constexpr (CENSUS) nin += (valid[0] && B.r2[u] <= A.rc2) ? 1u : 0u;
+                        float t;
+                        B.tb[u] = s_tab0[table_bin<LOGT>(B.r2[u], t, lam)];
+                    }
+                };
+                auto add = [&](const round& B) {
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const float f = fmaf(B.tb[u].y, B.r2[u], B.tb[u].x);
+                        ax[0] = fmaf(B.dx[u], f, ax[0]); ay[0] = fmaf(B.dy[u], f, ay[0]); az[0] = fmaf(B.dz[u], f, az[0]);
+                    }
+                };
+                load(0);
+                diff(P);
+                load(1);
+                look(P);
+#pragma unroll 1
+                for (int b = 1; b + 1 < NB; b += 2) {
+                    diff(Q);
+                    load(b + 1);
+                    look(Q);
+                    add(P);
+                    diff(P);
+                    load(b + 2);
+                    look(P);
+                    add(Q);
+                }
+                diff(Q);
+                look(Q);
+                add(P);
+                add(Q);
+            } else if constexpr (iters >= U) {
 #pragma unroll 2
                 for (int k = 0; k < iters; k += U) {
                     psrc s[U];
