@@ -1717,6 +1717,7 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f64_kernel(walk64_args A) {
         // lanes (slot, rep): slots x R of them, M targets each; three targets a lane where that uses
         // at least as many lanes, and for groups of more than 64
         const int s3 = (cnt + 2) / 3, R3 = 64 / s3, R1 = cnt <= 64 ? 64 / cnt : 0;
+        uint32_t next = 0u;
         auto group_body = [&](auto mc) {
             constexpr int M = decltype(mc)::value;
             const int slots = M == 3 ? s3 : cnt, R = M == 3 ? R3 : R1;
@@ -1940,6 +1941,9 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f64_kernel(walk64_args A) {
             for (int i = 0; i < M; i++) {
                 sx[lane] = ax[i]; sy[lane] = ay[i]; sz[lane] = az[i];
                 team_sync();
+                // The next group is read between the last two waits: the first wave writes the one after
+                // it only past the second of them, when every wave of the team has read this one.
+                if (i == M - 1) next = *(volatile uint32_t*)&s_next[team];
                 if (part == 0 && rep == 0 && valid[i]) {
                     double fx = 0.0, fy = 0.0, fz = 0.0;
                     for (int w = 0; w < S; w++)
@@ -1963,7 +1967,7 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f64_kernel(walk64_args A) {
         };
         if (R3 >= 3 * R1) group_body(ic<3>{});
         else group_body(ic<1>{});
-        g = (uint32_t)__builtin_amdgcn_readfirstlane((int)*(volatile uint32_t*)&s_next[team]);
+        g = (uint32_t)__builtin_amdgcn_readfirstlane((int)next);
     }
     if (lane == 0 && (npp | npc)) {
         atomicAdd(&A.counters[0], npp);
