@@ -745,7 +745,7 @@ int lagpm_pmmain(lagpm_ctx* ctx, lagpm_box* box, const lagpm_evolfact* ef, int p
     RCHK(pm_factor(ctx, ef, pmstatus, &f));
     hipEvent_t* ev = box->ev;
     HIPCHK(ctx, hipEventRecord(ev[0], box->st));
-    if (!box->sorted) RCHK(lagpm_sort_particles(ctx, box));
+    if (!lagpm_sorted_for_build(box)) RCHK(lagpm_sort_particles(ctx, box));
     HIPCHK(ctx, hipEventRecord(ev[1], box->st));
     HIPCHK(ctx, hipEventRecord(ev[12], box->st));
     RCHK(lagpm_pm_deposit(ctx, box));
@@ -822,7 +822,7 @@ int lagpm_force_spline(const lagpm_params* p, double* diff, double* slope) {
 static int tree_enqueue(lagpm_ctx* ctx, lagpm_box* box, double fact, bool combine) {
     hipEvent_t* ev = box->ev + 8;
     HIPCHK(ctx, hipEventRecord(ev[0], box->st));
-    if (!box->sorted) RCHK(lagpm_sort_particles(ctx, box));
+    if (!lagpm_sorted_for_build(box)) RCHK(lagpm_sort_particles(ctx, box));
     HIPCHK(ctx, hipEventRecord(ev[1], box->st));
     RCHK(lagpm_tree_build(ctx, box));
     HIPCHK(ctx, hipEventRecord(ev[2], box->st));
@@ -898,7 +898,7 @@ int lagpm_tree_accel_sample(lagpm_ctx* ctx, lagpm_box* box, const int64_t* ids, 
     // the box's tree, built as the tree correction builds it (grown or deepened as needed)
     for (int attempt = 0;; attempt++) {
         HIPCHK(ctx, hipEventRecord(box->ev[8], box->st));
-        if (!box->sorted) RCHK(lagpm_sort_particles(ctx, box));
+        if (!lagpm_sorted_for_build(box)) RCHK(lagpm_sort_particles(ctx, box));
         RCHK(lagpm_tree_build(ctx, box));
         bool retry = false;
         const int rc = lagpm_tree_finish(ctx, box, &retry);
@@ -1151,6 +1151,7 @@ void front_host_effects(lagpm_box* b) {
     std::swap(b->id, b->id_alt);
     b->parity ^= 1;
     b->sorted = true;
+    b->sorted_bits = lagpm_sort_bits(b);
 }
 
 // Everything of one box's step before the walk, queued on box->st (and box->st2), then the event

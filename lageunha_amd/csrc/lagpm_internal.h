@@ -126,6 +126,7 @@ struct lagpm_box {
     size_t bytes = 0;
     bool uploaded = false;
     bool sorted = false;
+    int sorted_bits = 0;      // leading key bits that the last sort put in order (any more are in no order)
     bool tree_built = false;  // a tree build has been queued (node arrays hold a tree)
     tree_tune tune;
     // deepest level the tree is expected to use: the full key depth until one build has run, then two
@@ -311,6 +312,9 @@ double lagpm_tree_scale(const lagpm_box* box);  // FP32 tree coordinate scale (s
 size_t lagpm_tree_node_cap_guess(size_t np, int mcell);
 size_t lagpm_tree_tmp_bytes(size_t np, size_t cap);  // scratch of a build of np particles into cap nodes
 int lagpm_choose_cell_level(int n, double rsphere);
+int lagpm_sort_bits(const lagpm_box* box);  // leading key bits that a sort of the box now puts in order
+// the last sort is still in force and ordered as many key bits as a build now relies on
+inline bool lagpm_sorted_for_build(const lagpm_box* box) { return box->sorted && box->sorted_bits >= lagpm_sort_bits(box); }
 size_t lagpm_walk_stack_entries(int num_cu);
 
 // ---- host helpers (api.hip) ----

@@ -2059,6 +2059,8 @@ static int build_depth(const lagpm_box* box) {
     return std::min(LAGPM_KEY_BITS, std::max(box->level_cell, box->depth));
 }
 
+int lagpm_sort_bits(const lagpm_box* box) { return 8 * sort_passes(box); }
+
 int lagpm_sort_particles(lagpm_ctx* ctx, lagpm_box* box, const double* drag, hipStream_t vst) {
     const size_t np = box->np;
     if (np == 0) return LAGPM_OK;
@@ -2098,6 +2100,7 @@ int lagpm_sort_particles(lagpm_ctx* ctx, lagpm_box* box, const double* drag, hip
     std::swap(box->id, box->id_alt);
     box->parity ^= 1;
     box->sorted = true;
+    box->sorted_bits = 8 * passes;
     return LAGPM_OK;
 }
 
@@ -2114,7 +2117,8 @@ int lagpm_tree_build(lagpm_ctx* ctx, lagpm_box* box) {
         HIPCHK(ctx, hipGetLastError());
         return LAGPM_OK;
     }
-    if (!box->sorted) RCHK(lagpm_sort_particles(ctx, box));
+    // (the depth limit may have been raised since the last sort: lagpm_box_set_tuning)
+    if (!lagpm_sorted_for_build(box)) RCHK(lagpm_sort_particles(ctx, box));
     const size_t ncell = (size_t)box->mcell * box->mcell * box->mcell;
     const int D = build_depth(box);
     const uint32_t nblk = (uint32_t)tree_part_blocks(np), gblk = (uint32_t)tree_group_blocks(cap);

@@ -1,0 +1,192 @@
+// host_runtime.cpp — the library's host code on a machine without a GPU: a stand-in for the HIP runtime
+// and rocFFT (device memory is host memory, copies are made at once, launched kernels are noted but not run),
+// and scenarios that look at what the host code queues. The program's definitions of the runtime's
+// functions come before the real runtime's. Usage: host_runtime SCENARIO; prints "name value" lines.
+#include <hip/hip_runtime_api.h>
+#include <rocfft/rocfft.h>
+
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <new>
+#include <string>
+#include <vector>
+
+#include "lagpm.h"
+
+struct ihipEvent_t {
+    size_t at = 0;
+};
+
+namespace {
+struct launch {
+    std::string kernel;
+    dim3 grid;
+};
+std::mutex mu;
+// the library registers its kernels before this program's own variables are set up
+std::map<const void*, std::string>& kernels() {
+    static auto* k = new std::map<const void*, std::string>;
+    return *k;
+}
+std::vector<launch> launches;
+dim3 call_grid, call_block;
+size_t call_lds;
+hipStream_t call_stream;
+char stream_mem[64];
+std::atomic<int> nstream{0};
+
+size_t count(const char* name) {  // launches so far of kernels of this name
+    std::lock_guard<std::mutex> lk(mu);
+    size_t c = 0;
+    for (const launch& l : launches) c += l.kernel.find(name) != std::string::npos;
+    return c;
+}
+}  // namespace
+
+extern "C" {
+void** __hipRegisterFatBinary(const void*) { return (void**)calloc(1, sizeof(void*)); }
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, dim3*, dim3*, int*) {
+    kernels()[host] = name;
+}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s) {
+    call_grid = g; call_block = b; call_lds = lds; call_stream = s;
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t* s) {
+    *g = call_grid; *b = call_block; *lds = call_lds; *s = call_stream;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void**, size_t, hipStream_t) {
+    std::lock_guard<std::mutex> lk(mu);
+    launches.push_back({kernels()[f], g});
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
+    memset(p, 0, sizeof(*p));
+    p->multiProcessorCount = 8;
+    return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "error of the stand-in"; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetSymbolAddress(void** p, const void*) { *p = calloc(1, 1 << 20); return hipSuccess; }
+hipError_t hipMalloc(void** p, size_t n) { *p = calloc(1, n); return hipSuccess; }
+hipError_t hipFree(void* p) { free(p); return hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = calloc(1, n); return hipSuccess; }
+hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { memset(d, v, n); return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)(stream_mem + nstream++); return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { *e = new ihipEvent_t; return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+    std::lock_guard<std::mutex> lk(mu);
+    e->at = launches.size();
+    return hipSuccess;
+}
+// "time" is the number of kernels queued between the two events
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
+    *ms = (float)((double)b->at - (double)a->at);
+    return hipSuccess;
+}
+
+rocfft_status rocfft_setup() { return rocfft_status_success; }
+rocfft_status rocfft_plan_description_create(rocfft_plan_description* d) { *d = (rocfft_plan_description)stream_mem; return rocfft_status_success; }
+rocfft_status rocfft_plan_description_destroy(rocfft_plan_description) { return rocfft_status_success; }
+rocfft_status rocfft_plan_description_set_data_layout(rocfft_plan_description, rocfft_array_type, rocfft_array_type, const size_t*,
+                                                      const size_t*, size_t, const size_t*, size_t, size_t, const size_t*, size_t) {
+    return rocfft_status_success;
+}
+rocfft_status rocfft_plan_create(rocfft_plan* p, rocfft_result_placement, rocfft_transform_type, rocfft_precision, size_t,
+                                 const size_t*, size_t, const rocfft_plan_description) {
+    *p = (rocfft_plan)stream_mem;
+    return rocfft_status_success;
+}
+rocfft_status rocfft_plan_destroy(rocfft_plan) { return rocfft_status_success; }
+rocfft_status rocfft_plan_get_work_buffer_size(const rocfft_plan, size_t* n) { *n = 0; return rocfft_status_success; }
+rocfft_status rocfft_execution_info_create(rocfft_execution_info* i) { *i = (rocfft_execution_info)stream_mem; return rocfft_status_success; }
+rocfft_status rocfft_execution_info_destroy(rocfft_execution_info) { return rocfft_status_success; }
+rocfft_status rocfft_execution_info_set_work_buffer(rocfft_execution_info, void*, size_t) { return rocfft_status_success; }
+rocfft_status rocfft_execution_info_set_stream(rocfft_execution_info, void*) { return rocfft_status_success; }
+rocfft_status rocfft_execute(const rocfft_plan, void**, void**, rocfft_execution_info) { return rocfft_status_success; }
+}
+
+namespace {
+lagpm_ctx* ctx;
+
+void must(int rc, const char* what) {
+    if (rc == LAGPM_OK) return;
+    printf("failed %s: %d %s\n", what, rc, lagpm_last_error(ctx));
+    exit(2);
+}
+#define MUST(call) must((call), #call)
+
+lagpm_params params(int n) {
+    lagpm_params p{};
+    p.n = n; p.law = LAGPM_LAW_ERFC; p.precision = LAGPM_PREC_FP32; p.deconvolve = 1;
+    p.mass = 1.0; p.efold = 2.5; p.epsilon = 0.1; p.rsphere = 5.625; p.theta = 0.5;
+    p.amax = 48.0; p.omep = 0.26; p.omeplam = 0.74;
+    return p;
+}
+lagpm_box* new_box(int n, size_t np) {
+    const lagpm_params p = params(n);
+    lagpm_box* b = nullptr;
+    MUST(lagpm_box_create(ctx, &p, np, &b));
+    const std::vector<double> x(np, 1.0);
+    MUST(lagpm_box_upload(ctx, b, x.data(), x.data(), x.data(), nullptr, nullptr, nullptr));
+    return b;
+}
+
+// Key bits in order: a build that may split deeper than the last sort's bits must sort again. Prints
+// the sorts queued by the tree correction in question.
+void resort() {
+    lagpm_evolfact ef{};
+    ef.fact1 = ef.fact2 = 1.0f;
+    lagpm_box* b = new_box(32, 1000);
+    MUST(lagpm_treecorrection(ctx, b, &ef));  // full sort; the (empty) tree's depth becomes the limit
+    MUST(lagpm_drift(ctx, b, 0.0));
+    MUST(lagpm_tsc(ctx, b, nullptr));  // sorts the bits of that limit
+    size_t before = count("keys_kernel");
+    MUST(lagpm_treecorrection(ctx, b, &ef));
+    printf("same_tuning %zu\n", count("keys_kernel") - before);
+    MUST(lagpm_box_set_tuning(b, 4, 8));  // the depth is to be found again
+    before = count("keys_kernel");
+    MUST(lagpm_treecorrection(ctx, b, &ef));
+    printf("other_tuning %zu\n", count("keys_kernel") - before);
+    before = count("keys_kernel");
+    MUST(lagpm_treecorrection(ctx, b, &ef));
+    printf("again %zu\n", count("keys_kernel") - before);
+    MUST(lagpm_drift(ctx, b, 0.0));
+    MUST(lagpm_tsc(ctx, b, nullptr));
+    before = count("keys_kernel");
+    MUST(lagpm_box_set_tuning(b, 16, 64));
+    const int64_t id = 0;
+    double acc[3];
+    MUST(lagpm_tree_accel_sample(ctx, b, &id, 1, acc));
+    printf("sample %zu\n", count("keys_kernel") - before);
+    MUST(lagpm_box_destroy(ctx, b));
+}
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::string what = argc > 1 ? argv[1] : "";
+    must(lagpm_create(&ctx, 0), "lagpm_create");
+    if (what == "resort") resort();
+    else return 3;
+    lagpm_destroy(ctx);
+    printf("end 0\n");
+    return 0;
+}

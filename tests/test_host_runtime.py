@@ -1,0 +1,35 @@
+"""The library's host code on the CPU, against a stand-in for the HIP runtime (host_runtime.cpp): what it
+queues, and how it fails."""
+import os
+import subprocess
+
+import pytest
+
+from lageunha_amd import lagpm
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+LIBDIR = os.path.dirname(lagpm.LIB_PATH)
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("host_runtime") / "host_runtime")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-rdynamic", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(os.path.dirname(HERE), "include"), os.path.join(HERE, "host_runtime.cpp"), "-o", out,
+                    "-L" + LIBDIR, "-llagpm", "-Wl,-rpath," + LIBDIR, "-Wl,-rpath-link,/opt/rocm/lib", "-pthread"], check=True)
+    return out
+
+
+def run(program, scenario, *args):
+    r = subprocess.run([program, scenario, *map(str, args)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, f"exit {r.returncode}: {r.stdout}{r.stderr}"
+    values = dict(line.split(" ", 1) for line in r.stdout.splitlines())
+    assert values.pop("end") == "0"
+    return {k: float(v) for k, v in values.items()}
+
+
+def test_a_build_deeper_than_the_sorted_key_bits_sorts_again(program):
+    """set_tuning puts the box's depth limit back to the full depth. The keys may have been sorted for
+    a shallower tree (here by tsc after a drift), and the build reads key order to the full depth."""
+    got = run(program, "resort")
+    assert got == {"same_tuning": 0, "other_tuning": 1, "again": 0, "sample": 1}
