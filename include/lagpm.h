@@ -330,11 +330,11 @@ int lagpm_kdk_step(lagpm_ctx* ctx, lagpm_box* box, double anow, double astep);
  * concurrently on a pool of streams, and the tree walks of all FP32 boxes with the same force
  * law run as one persistent launch. Each box's result equals its lagpm_kdk_step result. */
 int lagpm_batch_step(lagpm_ctx* ctx, lagpm_box* const* boxes, int nbox, const double* anow, const double* astep);
-/* On: whole steps capture each box's step (up to the tree walk) in a hipGraph on first use and
- * replay it. Off (default): every kernel is launched each step. Results are identical. Off because
- * a process that captured, launched and released many such graphs has ended in a segmentation fault
- * on the host now and then, and no cause has been shown. A call that turns them off also has the
- * steps that follow record their phase events (lagpm_box_timings). */
+/* Off: the steps that follow record their phase events (lagpm_box_timings); on, and without a call:
+ * they do not. Every kernel of a step is launched either way, with the same results. (A call that
+ * turned them on had steps replay captured hipGraphs. That was the slower path, and one process that
+ * captured and replayed many ended in a segmentation fault on the host, of which no cause was found:
+ * it has been taken out.) */
 int lagpm_set_step_graphs(lagpm_ctx* ctx, int enable);
 /* FP32 walks also count the evaluated particle pairs that are within the cutoff
  * (lagpm_tree_stats.n_pp_within): the useful fraction of the interaction lists. Costs a compare

@@ -37,7 +37,7 @@ __global__ void scatter_kernel(const double* __restrict__ src, const uint32_t* _
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < np) dst[id[i]] = src[i];
 }
-// kick factors live in device memory (box->dfac) so that a captured step reads this step's values
+// kick factors live in device memory (box->dfac), written by one small launch a step
 __global__ void set_factors_kernel(double* __restrict__ dfac, double f1, double f2, double pf, int mask) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     if (mask & 1) dfac[0] = f1;
@@ -129,7 +129,6 @@ void free_box(lagpm_box* b) {
     for (int a = 0; a < 6; a++) dfree(b->alt[a]);
     dfree(b->id_alt); dfree(b->dfac);
     lagpm_box_fft_release(b);
-    lagpm_box_graphs_release(b);
     dfree(b->acc); dfree(b->dep_start); dfree(b->rho); dfree(b->grad);
     b->spec = b->phi = nullptr;  // the same padded mesh as rho
     dfree(b->pp); dfree(b->nd_link); dfree(b->nd_lev); dfree(b->nd_rop); dfree(b->nd_geo); dfree(b->nd_q0); dfree(b->nd_q1);
@@ -571,10 +570,7 @@ static int upload_done(lagpm_ctx* ctx, lagpm_box* box) {
     // new particles: the box starts over as a new box would, with a full-depth first tree (the
     // depth limit also sets how many key bits the sort orders, and so the particle order that
     // the sums follow), so a box reused for other particles steps exactly as a fresh one
-    if (box->depth != LAGPM_KEY_BITS) {
-        box->depth = LAGPM_KEY_BITS;
-        lagpm_box_graphs_release(box);  // captured steps hold the old limit
-    }
+    box->depth = LAGPM_KEY_BITS;
     return LAGPM_OK;
 }
 
@@ -931,10 +927,8 @@ int lagpm_tree_accel_sample(lagpm_ctx* ctx, lagpm_box* box, const int64_t* ids, 
 
 int lagpm_box_set_tuning(lagpm_box* box, int nleaf, int group) {
     if (!box || nleaf < 4 || nleaf > 256 || group < 8 || group > 128) return LAGPM_E_INVAL;
-    if (box->tune.nleaf != nleaf || box->tune.group != group) {
-        lagpm_box_graphs_release(box);
+    if (box->tune.nleaf != nleaf || box->tune.group != group)
         box->depth = LAGPM_KEY_BITS;  // another leaf size: find the tree depth again
-    }
     box->tune.nleaf = nleaf;
     box->tune.group = group;
     return LAGPM_OK;
@@ -951,7 +945,6 @@ int lagpm_box_set_group_mode(lagpm_box* box, int mode) {
     if (!box || (mode != LAGPM_GROUPS_TREE && mode != LAGPM_GROUPS_RUNS && mode != LAGPM_GROUPS_PACKED))
         return LAGPM_E_INVAL;
     const int runs = mode == LAGPM_GROUPS_RUNS ? 1 : (mode == LAGPM_GROUPS_PACKED ? 2 : 0);
-    if (box->tune.runs != runs) lagpm_box_graphs_release(box);  // captured steps hold the mode
     box->tune.runs = runs;
     return LAGPM_OK;
 }
@@ -1091,10 +1084,8 @@ int ensure_pool(lagpm_ctx* ctx, size_t want) {
 // One box's step before the walk, queued on box->st with the factors already in box->dfac:
 // Hubble drag and sort, then a fork: the PM kick (deposit, FFTs, Green, gradient, interpolation)
 // on box->st beside the tree build on box->st2, joined on box->st. The PM branch is queued first:
-// a graph launch and an eager run both submit in queue order, and the build's many small kernels
-// would otherwise hold back the start of the longer PM chain. The build's latency-bound kernels
-// and the PM's memory-bound ones share the GPU. With ev: phase events (eager runs only; a capture
-// records none, but the fork and join events are part of it).
+// the build's many small kernels would otherwise hold back the start of the longer PM chain. The
+// build's latency-bound kernels and the PM's memory-bound ones share the GPU. With ev: phase events.
 int front_body(lagpm_ctx* ctx, lagpm_box* box, hipEvent_t* ev) {
     hipStream_t st = box->st, st2 = box->st2;
     if (ev) HIPCHK(ctx, hipEventRecord(ev[0], st));
@@ -1128,75 +1119,18 @@ int front_body(lagpm_ctx* ctx, lagpm_box* box, hipEvent_t* ev) {
     return LAGPM_OK;
 }
 
-struct box_ptrs {  // host-side pointer state a front changes (sort swaps)
-    double *x, *y, *z, *vx, *vy, *vz, *alt[6];
-    uint32_t *id, *id_alt;
-    int parity;
-    bool sorted;
-};
-box_ptrs save_ptrs(const lagpm_box* b) {
-    box_ptrs s{b->x, b->y, b->z, b->vx, b->vy, b->vz, {}, b->id, b->id_alt, b->parity, b->sorted};
-    for (int a = 0; a < 6; a++) s.alt[a] = b->alt[a];
-    return s;
-}
-void load_ptrs(lagpm_box* b, const box_ptrs& s) {
-    b->x = s.x; b->y = s.y; b->z = s.z; b->vx = s.vx; b->vy = s.vy; b->vz = s.vz;
-    for (int a = 0; a < 6; a++) b->alt[a] = s.alt[a];
-    b->id = s.id; b->id_alt = s.id_alt; b->parity = s.parity; b->sorted = s.sorted;
-}
-// what a front does to the host-side state, without queueing anything (graph replays)
-void front_host_effects(lagpm_box* b) {
-    std::swap(b->x, b->alt[0]); std::swap(b->y, b->alt[1]); std::swap(b->z, b->alt[2]);
-    std::swap(b->vx, b->alt[3]); std::swap(b->vy, b->alt[4]); std::swap(b->vz, b->alt[5]);
-    std::swap(b->id, b->id_alt);
-    b->parity ^= 1;
-    b->sorted = true;
-    b->sorted_bits = lagpm_sort_bits(b);
-}
-
 // Everything of one box's step before the walk, queued on box->st (and box->st2), then the event
-// the walk waits for (ev[13]). With step graphs turned on, the front is captured once per
-// particle-set parity and replayed; factors are written first.
+// the walk waits for (ev[13]); the step's factors are written first.
 int step_front(lagpm_ctx* ctx, lagpm_box* box, const lagpm_evolfact& ef) {
     hipLaunchKernelGGL(set_factors_kernel, dim3(1), dim3(64), 0, box->st, box->dfac, (double)ef.fact1, (double)ef.fact2,
                        (double)ef.pfact, 7);
     HIPCHK(ctx, hipGetLastError());
-    auto eager = [&]() -> int {
-        if (!ctx->step_events) {  // the events that every step's tree times need
-            HIPCHK(ctx, hipEventRecord(box->ev[8], box->st));
-            HIPCHK(ctx, hipEventRecord(box->ev[9], box->st));
-        }
-        RCHK(front_body(ctx, box, ctx->step_events ? box->ev : nullptr));
-        box->pm_timed = ctx->step_events;
-        HIPCHK(ctx, hipEventRecord(box->ev[13], box->st));
-        return LAGPM_OK;
-    };
-    if (!ctx->use_graphs || box->graph_failed) return eager();
-    // everything a capture must not do (plan creation and its check synchronise) happens first
-    RCHK(lagpm_pm_prepare(ctx, box));
-    HIPCHK(ctx, hipEventRecord(box->ev[8], box->st));
-    HIPCHK(ctx, hipEventRecord(box->ev[9], box->st));
-    hipGraphExec_t& ex = box->gfront[box->parity];
-    if (!ex) {
-        const box_ptrs before = save_ptrs(box);
-        hipGraph_t g = nullptr;
-        bool ok = hipStreamBeginCapture(box->st, hipStreamCaptureModeRelaxed) == hipSuccess;
-        int rc = ok ? front_body(ctx, box, nullptr) : LAGPM_E_HIP;
-        if (ok) ok = hipStreamEndCapture(box->st, &g) == hipSuccess && rc == LAGPM_OK && g;
-        if (ok) ok = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0) == hipSuccess;
-        if (g) (void)hipGraphDestroy(g);
-        load_ptrs(box, before);
-        (void)hipGetLastError();
-        if (!ok) {  // run eagerly from now on for this box
-            ex = nullptr;
-            box->graph_failed = true;
-            return eager();
-        }
+    if (!ctx->step_events) {  // the events that every step's tree times need
+        HIPCHK(ctx, hipEventRecord(box->ev[8], box->st));
+        HIPCHK(ctx, hipEventRecord(box->ev[9], box->st));
     }
-    HIPCHK(ctx, hipGraphLaunch(ex, box->st));
-    front_host_effects(box);
-    box->pm_timed = false;  // no phase events inside a graph
-    HIPCHK(ctx, hipEventRecord(box->ev[10], box->st));
+    RCHK(front_body(ctx, box, ctx->step_events ? box->ev : nullptr));
+    box->pm_timed = ctx->step_events;
     HIPCHK(ctx, hipEventRecord(box->ev[13], box->st));
     return LAGPM_OK;
 }
@@ -1415,14 +1349,6 @@ int batch_step(lagpm_ctx* ctx, lagpm_box* const* boxes, int nbox, const double* 
 
 }  // namespace
 
-void lagpm_box_graphs_release(lagpm_box* box) {
-    for (int q = 0; q < 2; q++)
-        if (box->gfront[q]) {
-            (void)hipGraphExecDestroy(box->gfront[q]);
-            box->gfront[q] = nullptr;
-        }
-}
-
 extern "C" {
 
 int lagpm_batch_step(lagpm_ctx* ctx, lagpm_box* const* boxes, int nbox, const double* anow, const double* astep) {
@@ -1431,7 +1357,6 @@ int lagpm_batch_step(lagpm_ctx* ctx, lagpm_box* const* boxes, int nbox, const do
 
 int lagpm_set_step_graphs(lagpm_ctx* ctx, int enable) {
     if (!ctx) return LAGPM_E_INVAL;
-    ctx->use_graphs = enable != 0;
     ctx->step_events = enable == 0;
     return LAGPM_OK;
 }

@@ -72,7 +72,6 @@ struct lagpm_ctx {
     walk_box* walk_boxes = nullptr;          // descriptor array of the last launch
     uint32_t* walk_prefix = nullptr;         // group prefix over the descriptors
     size_t walk_box_cap = 0;
-    bool use_graphs = false;                 // capture box step fronts in hipGraphs (lagpm_set_step_graphs)
     bool step_events = false;                // record the phase events of step fronts (lagpm_set_step_graphs(ctx, 0))
     bool walk_census = false;                // FP32 walks count the pairs within the cutoff
     int batch_stages = 0;                    // groups of a pipelined batch step (1: no pipeline; 0: by the boxes)
@@ -138,28 +137,23 @@ struct lagpm_box {
     hipStream_t st2 = nullptr;  // second stream of a step front (the tree build beside the PM kick)
 
     // particle state, kept in the current (sorted after a sort) order. A sort gathers into the
-    // other set and swaps the two, so the pointers alternate with period two (a captured step
-    // graph exists per parity).
+    // other set and swaps the two.
     double *x = nullptr, *y = nullptr, *z = nullptr, *vx = nullptr, *vy = nullptr, *vz = nullptr;
     uint32_t* id = nullptr;  // caller index of each particle
     double* alt[6] = {};     // the other set of x, y, z, vx, vy, vz
     uint32_t* id_alt = nullptr;
-    int parity = 0;
     // sort scratch
     uint64_t *key = nullptr, *key2 = nullptr;
     uint32_t *perm = nullptr, *perm2 = nullptr;
     // kick factors read by the kernels: [0] drag fact1, [1] PM kick factor, [2] drift pfact
     double* dfac = nullptr;
-    // FFT execution info and work buffer owned by the box (a captured graph refers to them)
+    // FFT execution info and work buffer owned by the box
     rocfft_execution_info fft_info = nullptr;
     void* fft_work = nullptr;
-    // captured front half of a step (drag .. tree build), one per particle-set parity
-    hipGraphExec_t gfront[2] = {nullptr, nullptr};  // captured step front per particle-set parity
     hipEvent_t evfork = nullptr;  // fork of the step front: the tree build branches off after the sort
     hipEvent_t evsort = nullptr;  // positions gathered: the velocity gather branches off
     hipEvent_t evvel = nullptr;   // velocities and ids gathered
     hipStream_t st3 = nullptr;    // the velocity gather's stream in a lone box's step front (else st)
-    bool graph_failed = false;
     uint32_t* scan_tmp = nullptr;  // scan / radix-sort scratch of this box (sort and tree build)
     size_t scan_tmp_bytes = 0;
     uint32_t* dep_scan_tmp = nullptr;  // the deposit's own scan scratch: it may run beside the tree build
@@ -258,7 +252,7 @@ int lagpm_pm_solve(lagpm_ctx* ctx, lagpm_box* box, hipEvent_t* ev = nullptr);  /
 int lagpm_pm_gradient(lagpm_ctx* ctx, lagpm_box* box);         // phi -> grad
 int lagpm_pm_interp(lagpm_ctx* ctx, lagpm_box* box);  // v += dfac[1] * F(grad)
 int lagpm_green_device(lagpm_ctx* ctx, hipStream_t s, int n, int prec, double efold, int deconvolve, void* spec);
-// the context's Green factor table for (n, efold, deconvolve); allocates (call before capture)
+// the context's Green factor table for (n, efold, deconvolve); the first call allocates
 int lagpm_green_prepare(lagpm_ctx* ctx, hipStream_t s, int n, double efold, int deconvolve);
 size_t lagpm_deposit_chunk_cap(int n, size_t np);
 size_t lagpm_deposit_blocks(int n);  // Morton blocks of the deposit's chunking
@@ -274,7 +268,6 @@ int lagpm_pm_power(lagpm_ctx* ctx, lagpm_box* box, double* pk_host, double* npk_
 int lagpm_pm_power_noalloc(lagpm_ctx* ctx, lagpm_box* box, double* pk_host, double* npk_host);
 // looks up (once per device, with the device current) the address of the static scratch
 int lagpm_pk_scratch_init(lagpm_ctx* ctx);
-void lagpm_box_graphs_release(lagpm_box* box);
 
 // ---- tree (tree.hip) ----
 // With vst (a stream other than box->st): the velocities and ids are gathered on vst, and

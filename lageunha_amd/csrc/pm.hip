@@ -901,8 +901,7 @@ __global__ void __launch_bounds__(256) pk_bin_kernel(const T* __restrict__ spec,
     }
 }
 
-// Plans (with their one-time check) and the box's execution info exist before a step is
-// captured: both synchronise or allocate, which a capture must not contain.
+// Makes the plans (with their one-time check), the box's execution info and the Green factor table.
 int lagpm_pm_prepare(lagpm_ctx* ctx, lagpm_box* box) {
     fft_plans* fp = nullptr;
     RCHK(get_plans(ctx, box->p.n, box->p.precision, box->st, &fp));
@@ -1129,7 +1128,7 @@ static double* green_table_find(lagpm_ctx* ctx, int n, double efold, int deconvo
 }
 
 // Makes the context's Green factor table for (n, efold, deconvolve) if the mesh is small enough
-// for one; allocates, so it runs before any captured step (lagpm_pm_prepare) or standalone call.
+// for one (the first call allocates).
 int lagpm_green_prepare(lagpm_ctx* ctx, hipStream_t st, int n, double efold, int deconvolve) {
     const size_t h = (size_t)n / 2 + 1, bytes = h * h * h * sizeof(double);
     if (bytes > GREEN_TAB_MAX_BYTES || green_table_find(ctx, n, efold, deconvolve)) return LAGPM_OK;
@@ -1180,7 +1179,6 @@ int lagpm_pm_solve(lagpm_ctx* ctx, lagpm_box* box, hipEvent_t* ev) {
     void* in[1] = {box->rho};  // rho, spec and phi are one padded mesh
     RCHK(fft_status(ctx, rocfft_execute(fp->fwd, in, nullptr, info), "execute(r2c)"));
     if (ev) HIPCHK(ctx, hipEventRecord(ev[0], box->st));
-    // (the table exists already when this runs inside a captured step: lagpm_pm_prepare made it)
     RCHK(lagpm_green_prepare(ctx, box->st, box->p.n, box->p.efold, box->p.deconvolve));
     RCHK(lagpm_green_device(ctx, box->st, box->p.n, box->p.precision, box->p.efold, box->p.deconvolve, box->spec));
     if (ev) HIPCHK(ctx, hipEventRecord(ev[1], box->st));

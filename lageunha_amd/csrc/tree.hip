@@ -877,8 +877,7 @@ __global__ void __launch_bounds__(GB_THREADS) group_write_kernel(const uint32_t*
     }
 }
 
-// start of a tree build: clear the size words and the interaction counters (a kernel, not a
-// memset, so the step can be captured in a graph)
+// an empty box's tree: clear the size words and the interaction counters
 __global__ void tree_reset_kernel(uint32_t* __restrict__ dsz, unsigned long long* __restrict__ counters) {
     tree_reset(threadIdx.x, dsz, counters);
 }
@@ -2017,7 +2016,6 @@ int lagpm_tree_alloc(lagpm_ctx* ctx, lagpm_box* box, size_t cap) {
             return lagpm_fail(ctx, LAGPM_E_INVAL, "tree needs more than 2^26 nodes (the walk's node index limit)");
         cap = LAGPM_MAX_NODES;
     }
-    lagpm_box_graphs_release(box);  // captured steps refer to the old arrays
     const size_t gcap = cap + box->np / 64 + 1;
     RCHK(regrow(ctx, &box->nd_link, cap));
     RCHK(regrow(ctx, &box->nd_lev, cap));
@@ -2042,8 +2040,8 @@ int lagpm_tree_alloc(lagpm_ctx* ctx, lagpm_box* box, size_t cap) {
 
 // The tree is expected to end above box->depth, so only the top 3 * depth key bits must be in order:
 // a box whose tree is shallower needs fewer passes. Below them the order is the previous one (the
-// sort is stable). An even number of passes leaves the result in key/perm, where captured steps and
-// the walk's descriptors expect it.
+// sort is stable). An even number of passes leaves the result in key/perm, where the gather and the
+// walk's descriptors expect it.
 static int sort_passes(const lagpm_box* box) {
     const int D = std::min(LAGPM_KEY_BITS, std::max(box->level_cell, box->depth));
     return (((3 * D + 7) / 8) + 1) & ~1;
@@ -2098,7 +2096,6 @@ int lagpm_sort_particles(lagpm_ctx* ctx, lagpm_box* box, const double* drag, hip
     HIPCHK(ctx, hipGetLastError());
     for (int a = 0; a < 6; a++) std::swap(*arrs[a], box->alt[a]);
     std::swap(box->id, box->id_alt);
-    box->parity ^= 1;
     box->sorted = true;
     box->sorted_bits = 8 * passes;
     return LAGPM_OK;
@@ -2284,7 +2281,6 @@ int lagpm_tree_finish_with(lagpm_ctx* ctx, lagpm_box* box, const tree_readback& 
         // nodes the truncated build could not count
         box->depth = LAGPM_KEY_BITS;
         box->sorted = false;  // the keys are in order down to the old limit only: sort again
-        lagpm_box_graphs_release(box);  // captured steps hold the old limit
         const size_t need = std::max<size_t>((size_t)d[DSZ_NODES], box->node_cap);
         if (d[DSZ_NODES] >= box->node_cap) RCHK(lagpm_tree_alloc(ctx, box, need + need / 2 + 4096));
         *retry = true;
@@ -2303,11 +2299,7 @@ int lagpm_tree_finish_with(lagpm_ctx* ctx, lagpm_box* box, const tree_readback& 
     box->stats.deepest = deepest;
     if (box->depth >= LAGPM_KEY_BITS) {
         // first complete build at full depth: limit later builds to two levels below its deepest
-        const int lim = std::min(LAGPM_KEY_BITS, deepest + 2);
-        if (lim < box->depth) {
-            box->depth = lim;
-            lagpm_box_graphs_release(box);  // captured steps hold the old limit
-        }
+        box->depth = std::min(LAGPM_KEY_BITS, deepest + 2);
     } else if (deepest > box->depth) {  // a build below the limit (build_depth): as a rebuild would set it
         box->depth = std::min(LAGPM_KEY_BITS, deepest + 2);
     }

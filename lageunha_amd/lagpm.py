@@ -229,6 +229,7 @@ class Context:
             raise LagpmError(rc, self.lib.lagpm_last_error(self.h).decode())
 
     def set_step_graphs(self, enable: bool):
+        """False: the steps that follow record their phase events (Box.timings)."""
         self.check(self.lib.lagpm_set_step_graphs(self.h, 1 if enable else 0))
 
     def set_walk_census(self, enable: bool):

@@ -38,6 +38,7 @@ size_t call_lds;
 hipStream_t call_stream;
 char stream_mem[64];
 std::atomic<int> nstream{0};
+std::atomic<int> ncapture{0};
 
 size_t count(const char* name) {  // launches so far of kernels of this name
     std::lock_guard<std::mutex> lk(mu);
@@ -88,6 +89,8 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { ncapture++; return hipErrorNotSupported; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return hipErrorNotSupported; }
 hipError_t hipEventCreate(hipEvent_t* e) { *e = new ihipEvent_t; return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
@@ -179,12 +182,28 @@ void resort() {
     printf("sample %zu\n", count("keys_kernel") - before);
     MUST(lagpm_box_destroy(ctx, b));
 }
+
+// Whole steps launch their kernels, whatever lagpm_set_step_graphs was told. The first one is left out: its
+// tree is built to the full depth, with a launch more a level.
+void steps() {
+    lagpm_box* b = new_box(32, 1000);
+    const int on[4] = {0, 1, 1, 0};
+    for (int i = 0; i < 4; i++) {
+        MUST(lagpm_set_step_graphs(ctx, on[i]));
+        const size_t before = launches.size();
+        MUST(lagpm_kdk_step(ctx, b, 1.0 + 0.1 * i, 0.1));
+        if (i) printf("step%d %zu\n", i, launches.size() - before);
+    }
+    printf("captures %d\n", ncapture.load());
+    MUST(lagpm_box_destroy(ctx, b));
+}
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     must(lagpm_create(&ctx, 0), "lagpm_create");
     if (what == "resort") resort();
+    else if (what == "steps") steps();
     else return 3;
     lagpm_destroy(ctx);
     printf("end 0\n");

@@ -33,3 +33,10 @@ def test_a_build_deeper_than_the_sorted_key_bits_sorts_again(program):
     a shallower tree (here by tsc after a drift), and the build reads key order to the full depth."""
     got = run(program, "resort")
     assert got == {"same_tuning": 0, "other_tuning": 1, "again": 0, "sample": 1}
+
+
+def test_steps_capture_no_graph(program):
+    """Whole steps queue the same kernels with set_step_graphs on and off, and capture nothing."""
+    got = run(program, "steps")
+    assert got.pop("captures") == 0
+    assert len(got) == 3 and len(set(got.values())) == 1 and min(got.values()) > 20
