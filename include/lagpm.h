@@ -122,6 +122,8 @@ typedef struct lagpm_timings {
 } lagpm_timings;
 
 /* ---- context --------------------------------------------------------------------- */
+/* A context's first copy of 2 MiB or more between the caller's memory and the device pins 64 MiB of
+ * host memory for all that follow, held until lagpm_destroy. */
 int         lagpm_create(lagpm_ctx** out, int device);
 int         lagpm_destroy(lagpm_ctx* ctx);
 const char* lagpm_last_error(const lagpm_ctx* ctx);

@@ -389,6 +389,7 @@ int lagpm_create(lagpm_ctx** out, int device) {
         return LAGPM_E_HIP;
     }
     for (int i = 0; i < 4; i++) (void)hipEventCreate(&ctx->ev[i]);
+    lagpm_stager_create(ctx);
     ctx->walk_stack_entries = lagpm_walk_stack_entries(ctx->num_cu);
     if (hipMalloc((void**)&ctx->walk_stack, ctx->walk_stack_entries * sizeof(int)) != hipSuccess ||
         hipMalloc((void**)&ctx->walk_ticket, LAGPM_WALK_XCDS * LAGPM_TICKET_STRIDE * sizeof(uint32_t)) != hipSuccess) {

@@ -85,7 +85,7 @@ struct lagpm_ctx {
     void* readback = nullptr;
     size_t readback_count = 0;
     void* readback1 = nullptr;
-    lagpm_stager* stager = nullptr;  // made by the first large host copy
+    lagpm_stager* stager = nullptr;  // null: no memory for it, large copies go the runtime's own way
 };
 
 // Tunables of the tree correction (chosen per box; the autotuner may override).
@@ -226,6 +226,7 @@ struct lagpm_segment {
     size_t bytes;
 };
 int lagpm_copy_segments(lagpm_ctx* ctx, const lagpm_segment* seg, size_t nseg, bool to_host, hipStream_t s);
+void lagpm_stager_create(lagpm_ctx* ctx);
 void lagpm_stager_release(lagpm_ctx* ctx);
 
 // ---- scans / sort (sort.hip) ----

@@ -114,8 +114,8 @@ int lagpm_copy_segments(lagpm_ctx* ctx, const lagpm_segment* seg, size_t nseg, b
     size_t total = 0;
     for (size_t k = 0; k < nseg; k++) total += seg[k].bytes;
     if (total < STAGED_MIN) return direct_copy(ctx, seg, nseg, to_host, st);
+    if (!ctx->stager) return direct_copy(ctx, seg, nseg, to_host, st);
     try {
-        if (!ctx->stager) ctx->stager = new lagpm_stager;
         lagpm_stager& S = *ctx->stager;
         std::lock_guard<std::mutex> lk(S.mu);
         if (!S.ready()) {  // no pinned memory to be had: the runtime's own path
@@ -158,6 +158,9 @@ int lagpm_h2d(lagpm_ctx* ctx, void* dst, const void* src, size_t bytes, hipStrea
     return lagpm_copy_segments(ctx, &g, 1, false, s);
 }
 
+// With the context, so that threads whose first copies come at once find the same one (and its lock); the
+// slots are pinned by the first large copy.
+void lagpm_stager_create(lagpm_ctx* ctx) { ctx->stager = new (std::nothrow) lagpm_stager; }
 void lagpm_stager_release(lagpm_ctx* ctx) {
     delete ctx->stager;
     ctx->stager = nullptr;

@@ -4,6 +4,7 @@
 // functions come before the real runtime's. Usage: host_runtime SCENARIO; prints "name value" lines.
 #include <hip/hip_runtime_api.h>
 #include <rocfft/rocfft.h>
+#include <unistd.h>
 
 #include <atomic>
 #include <cstdio>
@@ -13,6 +14,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "lagpm.h"
@@ -33,12 +35,13 @@ std::map<const void*, std::string>& kernels() {
     return *k;
 }
 std::vector<launch> launches;
-dim3 call_grid, call_block;
-size_t call_lds;
-hipStream_t call_stream;
+thread_local dim3 call_grid, call_block;
+thread_local size_t call_lds;
+thread_local hipStream_t call_stream;
 char stream_mem[64];
 std::atomic<int> nstream{0};
-std::atomic<int> ncapture{0};
+std::atomic<int> ncapture{0}, npinned{0};  // graph captures; pinned buffers of a megabyte and more
+thread_local int slow_new = 0;             // allocations of this thread take this many microseconds
 
 size_t count(const char* name) {  // launches so far of kernels of this name
     std::lock_guard<std::mutex> lk(mu);
@@ -47,6 +50,14 @@ size_t count(const char* name) {  // launches so far of kernels of this name
     return c;
 }
 }  // namespace
+
+void* operator new(size_t n) {
+    if (slow_new) usleep((useconds_t)slow_new);
+    if (void* p = malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 
 extern "C" {
 void** __hipRegisterFatBinary(const void*) { return (void**)calloc(1, sizeof(void*)); }
@@ -81,7 +92,11 @@ hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { *p = calloc(1, 1 << 20); return hipSuccess; }
 hipError_t hipMalloc(void** p, size_t n) { *p = calloc(1, n); return hipSuccess; }
 hipError_t hipFree(void* p) { free(p); return hipSuccess; }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = calloc(1, n); return hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    if (n >= 1 << 20) npinned++;
+    *p = calloc(1, n);
+    return hipSuccess;
+}
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { memset(d, v, n); return hipSuccess; }
@@ -197,6 +212,31 @@ void steps() {
     printf("captures %d\n", ncapture.load());
     MUST(lagpm_box_destroy(ctx, b));
 }
+
+// The first large copies of a context, by two threads at once on boxes of their own.
+void first_copies() {
+    const size_t np = 100000;  // three arrays of 0.8 MB: through the pinned slots
+    const lagpm_params p = params(32);
+    lagpm_box* b[2];
+    for (lagpm_box*& q : b) MUST(lagpm_box_create(ctx, &p, np, &q));
+    const std::vector<double> x(np, 1.0);
+    std::atomic<int> ready{0};
+    std::thread t[2];
+    int rc[2];
+    for (int i = 0; i < 2; i++)
+        t[i] = std::thread([&, i] {
+            ready++;
+            while (ready < 2) {}
+            slow_new = 20000;
+            rc[i] = lagpm_box_upload(ctx, b[i], x.data(), x.data(), x.data(), nullptr, nullptr, nullptr);
+            slow_new = 0;
+        });
+    for (std::thread& q : t) q.join();
+    must(rc[0], "upload of thread 0");
+    must(rc[1], "upload of thread 1");
+    printf("pinned %d\n", npinned.load());
+    for (lagpm_box* q : b) MUST(lagpm_box_destroy(ctx, q));
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -204,6 +244,7 @@ int main(int argc, char** argv) {
     must(lagpm_create(&ctx, 0), "lagpm_create");
     if (what == "resort") resort();
     else if (what == "steps") steps();
+    else if (what == "first_copies") first_copies();
     else return 3;
     lagpm_destroy(ctx);
     printf("end 0\n");

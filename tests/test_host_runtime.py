@@ -40,3 +40,8 @@ def test_steps_capture_no_graph(program):
     got = run(program, "steps")
     assert got.pop("captures") == 0
     assert len(got) == 3 and len(set(got.values())) == 1 and min(got.values()) > 20
+
+
+def test_first_copies_of_two_threads_share_one_set_of_slots(program):
+    """Two threads make a context's first large copies at once: one set of pinned slots is made for them."""
+    assert run(program, "first_copies") == {"pinned": 1}
