@@ -8,8 +8,8 @@
 // ms, up and down again 51 -> 22.5 ms.
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <new>
-#include <system_error>
 #include <thread>
 
 #include "lagpm_internal.h"
@@ -134,7 +134,7 @@ int lagpm_copy_segments(lagpm_ctx* ctx, const lagpm_segment* seg, size_t nseg, b
         for (int w = 1; w < workers; w++) {
             try {
                 others[w] = std::thread([&, w] { S.work(w, ctx->device, chunks, next, err, to_host, st); });
-            } catch (const std::system_error&) {  // no thread to be had: the others take its chunks
+            } catch (const std::exception&) {  // no thread or no memory for one: the others take its chunks
                 break;
             }
         }

@@ -41,7 +41,15 @@ thread_local hipStream_t call_stream;
 char stream_mem[64];
 std::atomic<int> nstream{0};
 std::atomic<int> ncapture{0}, npinned{0};  // graph captures; pinned buffers of a megabyte and more
+std::atomic<size_t> nuploaded{0};          // bytes copied to the device
 thread_local int slow_new = 0;             // allocations of this thread take this many microseconds
+thread_local int fail_new = 0;             // the fail_new-th allocation of this thread from here on fails
+
+struct own {  // the stand-in's own allocations neither fail nor count
+    int f = fail_new;
+    own() { fail_new = 0; }
+    ~own() { fail_new = f; }
+};
 
 size_t count(const char* name) {  // launches so far of kernels of this name
     std::lock_guard<std::mutex> lk(mu);
@@ -53,6 +61,7 @@ size_t count(const char* name) {  // launches so far of kernels of this name
 
 void* operator new(size_t n) {
     if (slow_new) usleep((useconds_t)slow_new);
+    if (fail_new && --fail_new == 0) throw std::bad_alloc();
     if (void* p = malloc(n ? n : 1)) return p;
     throw std::bad_alloc();
 }
@@ -75,6 +84,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
     return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void**, size_t, hipStream_t) {
+    own quiet;
     std::lock_guard<std::mutex> lk(mu);
     launches.push_back({kernels()[f], g});
     return hipSuccess;
@@ -98,7 +108,11 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
     return hipSuccess;
 }
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, hipStream_t) {
+    memcpy(d, s, n);
+    if (kind == hipMemcpyHostToDevice) nuploaded += n;
+    return hipSuccess;
+}
 hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { memset(d, v, n); return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)(stream_mem + nstream++); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
@@ -106,7 +120,7 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { ncapture++; return hipErrorNotSupported; }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return hipErrorNotSupported; }
-hipError_t hipEventCreate(hipEvent_t* e) { *e = new ihipEvent_t; return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { own quiet; *e = new ihipEvent_t; return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
@@ -237,6 +251,27 @@ void first_copies() {
     printf("pinned %d\n", npinned.load());
     for (lagpm_box* q : b) MUST(lagpm_box_destroy(ctx, q));
 }
+
+// A large copy with each allocation that it makes on the host failing in turn: it says so, or does
+// without, and a copy that reports success has moved every byte.
+void no_host_memory() {
+    const size_t np = 1000000;
+    const lagpm_params p = params(32);
+    lagpm_box* b = nullptr;
+    MUST(lagpm_box_create(ctx, &p, np, &b));
+    const std::vector<double> x(np, 1.0);
+    int refused = 0, done = 0, other = 0, partial = 0;
+    for (int k = 1; k <= 40; k++) {
+        const size_t before = nuploaded;
+        fail_new = k;
+        const int rc = lagpm_box_upload(ctx, b, x.data(), x.data(), x.data(), nullptr, nullptr, nullptr);
+        fail_new = 0;
+        (rc == LAGPM_OK ? done : rc == LAGPM_E_NOMEM ? refused : other)++;
+        if (rc == LAGPM_OK && nuploaded - before != 3 * np * sizeof(double)) partial++;
+    }
+    printf("refused %d\ndone_some %d\nother %d\npartial %d\n", refused > 0, done > 20, other, partial);
+    MUST(lagpm_box_destroy(ctx, b));
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -245,6 +280,7 @@ int main(int argc, char** argv) {
     if (what == "resort") resort();
     else if (what == "steps") steps();
     else if (what == "first_copies") first_copies();
+    else if (what == "no_host_memory") no_host_memory();
     else return 3;
     lagpm_destroy(ctx);
     printf("end 0\n");

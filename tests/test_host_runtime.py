@@ -45,3 +45,9 @@ def test_steps_capture_no_graph(program):
 def test_first_copies_of_two_threads_share_one_set_of_slots(program):
     """Two threads make a context's first large copies at once: one set of pinned slots is made for them."""
     assert run(program, "first_copies") == {"pinned": 1}
+
+
+def test_large_copy_without_host_memory(program):
+    """Each host allocation of a large copy fails in turn (the chunk list, the threads' states): the copy
+    returns, with LAGPM_E_NOMEM or complete, and the process goes on."""
+    assert run(program, "no_host_memory") == {"refused": 1, "done_some": 1, "other": 0, "partial": 0}
