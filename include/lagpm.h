@@ -97,7 +97,7 @@ typedef struct lagpm_tree_stats {
     uint64_t n_pc;      /* particle-node (quadrupole) pairs evaluated */
     uint64_t n_nodes;   /* octree nodes built */
     uint64_t n_groups;  /* target groups walked */
-    double   ms_build;  /* sort + build + moments, device time */
+    double   ms_build;  /* build + moments + groups, and the sort where treecorrection made one; device time */
     double   ms_walk;   /* walk kernel, device time */
     int32_t  deepest;   /* deepest tree level with nodes (levels of the 16-bit-per-axis keys) */
     int32_t  depth_limit; /* deepest level the next tree is expected to use (a deeper one is detected
@@ -117,7 +117,7 @@ typedef struct lagpm_timings {
     double ms_grad;     /* FDA4 gradient mesh */
     double ms_interp;   /* TSC interpolation + kick (with ms_grad: CPU(4FDA)) */
     double ms_tree_sort;/* sort inside treecorrection (0 when pmmain already sorted) */
-    double ms_build;    /* octree build + moments + groups */
+    double ms_build;    /* octree build + moments + groups (of whole steps too) */
     double ms_walk;     /* walk + kick (CPU(TREE) with ms_build) */
 } lagpm_timings;
 

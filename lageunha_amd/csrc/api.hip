@@ -839,7 +839,7 @@ static int tree_enqueue(lagpm_ctx* ctx, lagpm_box* box, double fact, bool combin
             HIPCHK(ctx, hipGetLastError());
         }
     }
-    box->tree_timed = true;
+    box->tree_timed = box->tree_sort_timed = true;
     return LAGPM_OK;
 }
 
@@ -847,7 +847,7 @@ static void tree_times(lagpm_box* box) {
     hipEvent_t* ev = box->ev + 8;
     float t01 = 0, t12 = 0, t23 = 0;
     (void)hipEventSynchronize(ev[3]);
-    (void)hipEventElapsedTime(&t01, ev[0], ev[1]);
+    if (box->tree_sort_timed) (void)hipEventElapsedTime(&t01, ev[0], ev[1]);
     (void)hipEventElapsedTime(&t12, ev[1], ev[2]);
     (void)hipEventElapsedTime(&t23, box->ev[14], ev[3]);  // walk start .. walk end
     box->stats.ms_build = t01 + t12;
@@ -1020,7 +1020,7 @@ int lagpm_box_timings(lagpm_ctx* ctx, lagpm_box* box, lagpm_timings* out) {
         out->ms_interp = el(6, 7);
     }
     if (box->tree_timed) {
-        out->ms_tree_sort = el(8, 9);
+        out->ms_tree_sort = box->tree_sort_timed ? el(8, 9) : 0.0;
         out->ms_build = el(9, 10);
         out->ms_walk = el(14, 11);  // from right before the walk launch to its end
     }
@@ -1086,7 +1086,8 @@ int ensure_pool(lagpm_ctx* ctx, size_t want) {
 // Hubble drag and sort, then a fork: the PM kick (deposit, FFTs, Green, gradient, interpolation)
 // on box->st beside the tree build on box->st2, joined on box->st. The PM branch is queued first:
 // the build's many small kernels would otherwise hold back the start of the longer PM chain. The
-// build's latency-bound kernels and the PM's memory-bound ones share the GPU. With ev: phase events.
+// build's latency-bound kernels and the PM's memory-bound ones share the GPU. With ev: the phase events
+// of the sort and the PM kick as well.
 int front_body(lagpm_ctx* ctx, lagpm_box* box, hipEvent_t* ev) {
     hipStream_t st = box->st, st2 = box->st2;
     if (ev) HIPCHK(ctx, hipEventRecord(ev[0], st));
@@ -1107,10 +1108,8 @@ int front_body(lagpm_ctx* ctx, lagpm_box* box, hipEvent_t* ev) {
     if (ev) HIPCHK(ctx, hipEventRecord(ev[7], st));
     const bool fork = st2 != st;  // several boxes in a batch build on their own streams
     if (fork) HIPCHK(ctx, hipStreamWaitEvent(st2, box->evfork, 0));
-    if (ev) {
-        HIPCHK(ctx, hipEventRecord(ev[8], st2));
-        HIPCHK(ctx, hipEventRecord(ev[9], st2));  // sorted above: no tree sort
-    }
+    HIPCHK(ctx, hipEventRecord(box->ev[9], st2));  // every step has its build timed
+    box->tree_sort_timed = false;                  // sorted above
     box->st = st2;
     const int rb = lagpm_tree_build(ctx, box);
     box->st = st;
@@ -1126,10 +1125,6 @@ int step_front(lagpm_ctx* ctx, lagpm_box* box, const lagpm_evolfact& ef) {
     hipLaunchKernelGGL(set_factors_kernel, dim3(1), dim3(64), 0, box->st, box->dfac, (double)ef.fact1, (double)ef.fact2,
                        (double)ef.pfact, 7);
     HIPCHK(ctx, hipGetLastError());
-    if (!ctx->step_events) {  // the events that every step's tree times need
-        HIPCHK(ctx, hipEventRecord(box->ev[8], box->st));
-        HIPCHK(ctx, hipEventRecord(box->ev[9], box->st));
-    }
     RCHK(front_body(ctx, box, ctx->step_events ? box->ev : nullptr));
     box->pm_timed = ctx->step_events;
     HIPCHK(ctx, hipEventRecord(box->ev[13], box->st));

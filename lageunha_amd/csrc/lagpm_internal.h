@@ -197,7 +197,7 @@ struct lagpm_box {
     // phase events: [0..7] pmmain (start, sort, tsc, r2c, green, c2r, grad, interp),
     //               [8..11] treecorrection (start, sort, build, walk)
     hipEvent_t ev[15] = {};  // phase events; [12] deposit start, [13] step front joined, [14] walk start
-    bool pm_timed = false, tree_timed = false;
+    bool pm_timed = false, tree_timed = false, tree_sort_timed = false;
 };
 
 // ---- error helpers ----

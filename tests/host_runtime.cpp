@@ -272,6 +272,26 @@ void no_host_memory() {
     printf("refused %d\ndone_some %d\nother %d\npartial %d\n", refused > 0, done > 20, other, partial);
     MUST(lagpm_box_destroy(ctx, b));
 }
+
+// The tree times of a step cover the tree build alone, with the other phases' events recorded or not,
+// for one box and for boxes of a batch.
+void build_times() {
+    lagpm_box* b[3] = {new_box(32, 1000), new_box(32, 1000), new_box(32, 1000)};
+    const double a[3] = {1.0, 1.0, 1.0}, da[3] = {0.1, 0.1, 0.1};
+    for (lagpm_box* q : b) MUST(lagpm_kdk_step(ctx, q, 1.0, 0.1));  // (full depth the first time)
+    for (int events : {0, 1}) {
+        MUST(lagpm_set_step_graphs(ctx, !events));
+        for (int nbox : {1, 3}) {
+            MUST(lagpm_batch_step(ctx, b, nbox, a, da));
+            lagpm_timings t;
+            lagpm_tree_stats s;
+            MUST(lagpm_box_timings(ctx, b[0], &t));
+            MUST(lagpm_tree_stats_get(b[0], &s));
+            printf("events%d_boxes%d_timings %g\nevents%d_boxes%d_stats %g\n", events, nbox, t.ms_build, events, nbox, s.ms_build);
+        }
+    }
+    for (lagpm_box* q : b) MUST(lagpm_box_destroy(ctx, q));
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -281,6 +301,7 @@ int main(int argc, char** argv) {
     else if (what == "steps") steps();
     else if (what == "first_copies") first_copies();
     else if (what == "no_host_memory") no_host_memory();
+    else if (what == "build_times") build_times();
     else return 3;
     lagpm_destroy(ctx);
     printf("end 0\n");

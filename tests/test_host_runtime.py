@@ -51,3 +51,10 @@ def test_large_copy_without_host_memory(program):
     """Each host allocation of a large copy fails in turn (the chunk list, the threads' states): the copy
     returns, with LAGPM_E_NOMEM or complete, and the process goes on."""
     assert run(program, "no_host_memory") == {"refused": 1, "done_some": 1, "other": 0, "partial": 0}
+
+
+def test_build_times_cover_the_build_alone(program):
+    """ms_build of a step is the octree build (here counted in its kernels: 3 for the nodes, one a level for the
+    moments, 3 for the groups), without the sort and the PM kick, whether phase events are recorded or not."""
+    got = run(program, "build_times")
+    assert len(got) == 8 and len(set(got.values())) == 1 and 7 <= min(got.values()) <= 11
