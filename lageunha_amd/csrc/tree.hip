@@ -2017,6 +2017,7 @@ int lagpm_tree_alloc(lagpm_ctx* ctx, lagpm_box* box, size_t cap) {
         cap = LAGPM_MAX_NODES;
     }
     const size_t gcap = cap + box->np / 64 + 1;
+    box->node_cap = box->group_cap = 0;  // none until all are there: the old arrays go first
     RCHK(regrow(ctx, &box->nd_link, cap));
     RCHK(regrow(ctx, &box->nd_lev, cap));
     RCHK(regrow(ctx, &box->nd_rop, cap));
@@ -2029,8 +2030,11 @@ int lagpm_tree_alloc(lagpm_ctx* ctx, lagpm_box* box, size_t cap) {
         RCHK(regrow(ctx, &box->nd_q1, cap));
     }
     const size_t need = std::max(lagpm_tree_tmp_bytes(box->np, cap), lagpm_sort_tmp_bytes(box->np));
-    if (need > box->scan_tmp_bytes) {
-        RCHK(regrow(ctx, (char**)&box->scan_tmp, need));
+    if (need > box->scan_tmp_bytes) {  // (small; sorts go on with the old one if this fails)
+        uint32_t* tmp = nullptr;
+        RCHK(regrow(ctx, (char**)&tmp, need));
+        if (box->scan_tmp) (void)hipFree(box->scan_tmp);
+        box->scan_tmp = tmp;
         box->scan_tmp_bytes = need;
     }
     box->node_cap = cap;
@@ -2108,6 +2112,8 @@ int lagpm_tree_build(lagpm_ctx* ctx, lagpm_box* box) {
     const int G = box->tune.group;
     const bool f64 = box->p.precision == LAGPM_PREC_FP64;
     hipStream_t st = box->st;
+    // an earlier growth of the node arrays failed and left none
+    if (box->node_cap == 0) RCHK(lagpm_tree_alloc(ctx, box, lagpm_tree_node_cap_guess(np, box->mcell)));
     const size_t cap = box->node_cap, gcap = box->group_cap;
     if (np == 0) {
         hipLaunchKernelGGL(tree_reset_kernel, dim3(1), dim3(64), 0, st, box->dsz, box->counters);
@@ -2171,6 +2177,7 @@ int lagpm_tree_walk_f32(lagpm_ctx* ctx, lagpm_box* const* boxes, const double* f
     if (sample && nbox != 1) return lagpm_fail(ctx, LAGPM_E_INVAL, "a sampled walk takes one box");
     if ((size_t)nbox > ctx->walk_box_cap) {
         size_t cap = std::max<size_t>(64, (size_t)nbox * 2);
+        ctx->walk_box_cap = 0;
         RCHK(regrow(ctx, &ctx->walk_boxes, cap));
         RCHK(regrow(ctx, &ctx->walk_prefix, cap + 1));
         ctx->walk_box_cap = cap;

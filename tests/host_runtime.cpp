@@ -42,6 +42,8 @@ char stream_mem[64];
 std::atomic<int> nstream{0};
 std::atomic<int> ncapture{0}, npinned{0};  // graph captures; pinned buffers of a megabyte and more
 std::atomic<size_t> nuploaded{0};          // bytes copied to the device
+uint32_t plant_nodes = 0;                  // tree builds find this many nodes, and that they do not fit
+int malloc_fails = 0, nbad = 0;            // device allocations fail; launches of empty grids or with null node arrays
 thread_local int slow_new = 0;             // allocations of this thread take this many microseconds
 thread_local int fail_new = 0;             // the fail_new-th allocation of this thread from here on fails
 
@@ -83,10 +85,20 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
     *g = call_grid; *b = call_block; *lds = call_lds; *s = call_stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void**, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void** args, size_t, hipStream_t) {
     own quiet;
     std::lock_guard<std::mutex> lk(mu);
     launches.push_back({kernels()[f], g});
+    const std::string& name = launches.back().kernel;
+    auto pointer = [&](int i) { return *(void**)args[i]; };
+    if (g.x == 0 || g.y == 0 || g.z == 0) nbad++;
+    if (name.find("tree_rows_kernel") != std::string::npos) {  // (sizes: nodes first, overflow fourth)
+        ((uint32_t*)pointer(5))[0] = plant_nodes;
+        ((uint32_t*)pointer(5))[3] = plant_nodes ? 1u : 0u;
+    }
+    if (name.find("tree_emit_kernel") != std::string::npos)  // the node arrays that it writes
+        for (int i : {5, 8, 9, 10, 11, 12})
+            if (!pointer(i)) nbad++;
     return hipSuccess;
 }
 hipError_t hipSetDevice(int) { return hipSuccess; }
@@ -100,7 +112,11 @@ hipError_t hipDeviceSynchronize() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "error of the stand-in"; }
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { *p = calloc(1, 1 << 20); return hipSuccess; }
-hipError_t hipMalloc(void** p, size_t n) { *p = calloc(1, n); return hipSuccess; }
+hipError_t hipMalloc(void** p, size_t n) {
+    if (malloc_fails) return hipErrorOutOfMemory;
+    *p = calloc(1, n);
+    return hipSuccess;
+}
 hipError_t hipFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
     if (n >= 1 << 20) npinned++;
@@ -292,9 +308,38 @@ void build_times() {
     }
     for (lagpm_box* q : b) MUST(lagpm_box_destroy(ctx, q));
 }
+
+// Node arrays that cannot be grown: the call fails, and later ones find arrays or make them.
+void no_device_memory() {
+    lagpm_evolfact ef{};
+    ef.fact1 = ef.fact2 = 1.0f;
+    lagpm_box* b = new_box(32, 1000);
+    MUST(lagpm_treecorrection(ctx, b, &ef));
+    plant_nodes = 100000;
+    malloc_fails = 1;
+    printf("grow %d\n", lagpm_treecorrection(ctx, b, &ef) != LAGPM_OK);
+    plant_nodes = 0;
+    printf("still_none %d\n", lagpm_treecorrection(ctx, b, &ef) != LAGPM_OK);
+    malloc_fails = 0;
+    printf("again %d\n", lagpm_treecorrection(ctx, b, &ef));
+    // the descriptors of a walk over many boxes
+    const std::vector<double> a(70, 1.0), da(70, 0.1);
+    std::vector<lagpm_box*> many;
+    for (int i = 0; i < 70; i++) many.push_back(new_box(24, 10));
+    MUST(lagpm_set_batch_pipeline(ctx, 1, 0));
+    MUST(lagpm_batch_step(ctx, many.data(), 2, a.data(), da.data()));
+    malloc_fails = 1;
+    printf("many %d\n", lagpm_batch_step(ctx, many.data(), 70, a.data(), da.data()) != LAGPM_OK);
+    malloc_fails = 0;
+    printf("many_again %d\n", lagpm_batch_step(ctx, many.data(), 2, a.data(), da.data()));
+    printf("bad_launches %d\n", nbad);
+    for (lagpm_box* q : many) MUST(lagpm_box_destroy(ctx, q));
+    MUST(lagpm_box_destroy(ctx, b));
+}
 }  // namespace
 
 int main(int argc, char** argv) {
+    setvbuf(stdout, nullptr, _IONBF, 0);
     const std::string what = argc > 1 ? argv[1] : "";
     must(lagpm_create(&ctx, 0), "lagpm_create");
     if (what == "resort") resort();
@@ -302,6 +347,7 @@ int main(int argc, char** argv) {
     else if (what == "first_copies") first_copies();
     else if (what == "no_host_memory") no_host_memory();
     else if (what == "build_times") build_times();
+    else if (what == "no_device_memory") no_device_memory();
     else return 3;
     lagpm_destroy(ctx);
     printf("end 0\n");

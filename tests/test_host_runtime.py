@@ -58,3 +58,10 @@ def test_build_times_cover_the_build_alone(program):
     moments, 3 for the groups), without the sort and the PM kick, whether phase events are recorded or not."""
     got = run(program, "build_times")
     assert len(got) == 8 and len(set(got.values())) == 1 and 7 <= min(got.values()) <= 11
+
+
+def test_node_arrays_that_cannot_be_grown(program):
+    """The growth of the node arrays (or of the walk's descriptors) fails for lack of device memory: that
+    call fails, and the calls after it launch nothing on the arrays that were given up."""
+    got = run(program, "no_device_memory")
+    assert got == {"grow": 1, "still_none": 1, "again": 0, "many": 1, "many_again": 0, "bad_launches": 0}
