@@ -12,7 +12,7 @@ One step = one GOTPM step through the C ABI's whole-step entry point (lagpm_kdk_
 drag, PM kick, tree kick, drift, in the reference's order (Cosmos/globalT.c:221-306). The sort,
 tree build and every kernel run inside every step; the PM kick runs beside the tree walk.
 value = particles / step time = TreePM forces/s (one force evaluation per step). Per-phase
-device times come from two more steps launched eagerly after the timed ones.
+device times come from two more steps with phase events after the timed ones.
 
 Printed: one JSON line (rank 0) with roofline (dominant kernel, live HIP-event durations),
 cpu_baseline (the CPU oracle on a bounded sample), accuracy vs the plain FP64 kernels.
@@ -289,14 +289,6 @@ def ensemble(args, ctx, lagpm, ics):
         lat["batched"].append(time.perf_counter() - t)
     tt["batched"] = time.perf_counter() - t0
     log(f"[bench] ensemble batched: {tt['batched']:.2f} s")
-    # two more batched steps: every kernel is launched in these as in the ones above (no step graphs)
-    t0 = time.perf_counter()
-    for s in range(2):
-        lagpm.batch_step(ctx, sets["batched"], a0 + da * (steps + 1 + s), da)
-    t_eager = (time.perf_counter() - t0) / 2
-    for s in range(2):  # keep the plain set in step with the batched one
-        for bx in sets["plain"]:
-            bx.kdk_step(a0 + da * (steps + 1 + s), da)
     same = True
     for bp, bb in zip(sets["plain"], sets["batched"]):
         xp, vp = bp.download()
@@ -317,7 +309,6 @@ def ensemble(args, ctx, lagpm, ics):
                   "step_latency_p50_ms": float(np.percentile(L, 50)), "step_latency_p99_ms": float(np.percentile(L, 99)),
                   "latency_unit": "one box-step (plain) / one batch step of all boxes (batched)"}
     out["batched_over_plain"] = out["batched"]["particle_steps_per_s"] / out["plain"]["particle_steps_per_s"]
-    out["batched_without_graphs"] = {"particle_steps_per_s": total / t_eager, "step_ms": t_eager * 1e3}
     # the plain FP64 kernels, box by box (one step each after a warm-up step)
     t_fp64, ps = 0.0, 0
     for b, (n, om) in enumerate(specs):
@@ -528,6 +519,7 @@ def main():
         phases.append(box.timings().as_dict())
         s = box.tree_stats()
         stats.append((s.n_pp, s.n_pc, s.n_nodes, s.n_groups))
+    ctx.set_step_graphs(True)  # the default: no phase events
     # one more step with the walk counting the evaluated pairs within the cutoff (slower, untimed)
     ctx.set_walk_census(True)
     step()

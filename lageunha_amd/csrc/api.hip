@@ -1185,9 +1185,11 @@ int batch_step(lagpm_ctx* ctx, lagpm_box* const* boxes, int nbox, const double* 
     // drift is queued after all fronts, so no front waits behind a walk on its pool stream.
     // Where the caller has not set the stages: up to five, about four boxes per group. A group's
     // walk ends with its heaviest target groups, which many boxes hide and few do not. ms per step at
-    // 1 / 2 / 3 / 4 / 5 stages: 8 boxes of 32^3-96^3 4.36 4.68 4.91 5.19 5.24; 10 of them 5.78 5.39 5.05
-    // 5.29 5.55; 16 of them 7.76 8.13 7.79 7.87 7.85; 20 of them 10.3 9.58 9.62 9.37 9.43; 14 of
-    // 32^3-64^3 4.93 4.89 4.35 4.58 4.86; 30 of 32^3-64^3 8.75 8.64 8.44 8.25 8.01.
+    // 1 / 2 / 3 / 4 / 5 stages, the rule's choice in brackets: 8 boxes of 32^3-96^3 4.36 [4.68] 4.91
+    // 5.19 5.24; 10 of them 5.78 5.39 [5.05] 5.29 5.55; 16 of them 7.76 8.13 7.79 [7.87] 7.85; 20 of
+    // them 10.3 9.58 9.62 9.37 [9.43]; 14 of 32^3-64^3 4.93 4.89 4.35 [4.58] 4.86; 30 of 32^3-64^3
+    // 8.75 8.64 8.44 8.25 [8.01]. It is within 8 % of the best count everywhere and level with or ahead of five,
+    // taken for all before; a rule on the cost of the walks' tails would come closer.
     int stages = ctx->batch_stages ? std::min<int>(ctx->batch_stages, (int)(live.size() / 2))
                                    : std::min<int>(5, (int)((live.size() + 2) / 4));
     for (lagpm_box* b : live)

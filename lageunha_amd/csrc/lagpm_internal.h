@@ -218,7 +218,8 @@ int lagpm_fail(lagpm_ctx* ctx, int code, const std::string& msg);
 // the outcome: the stream is synchronised even when queuing the copy fails, so no copy can still
 // be writing into host memory the caller is about to free or leave (stack buffers included).
 int lagpm_d2h(lagpm_ctx* ctx, void* dst, const void* src, size_t bytes, hipStream_t s);
-// Host-to-device copy queued on stream s; the host memory is the caller's again when it returns.
+// Host-to-device copy queued on stream s. The host memory is the caller's again when the stream has been
+// waited for (a copy from pinned memory is still under way when this returns).
 int lagpm_h2d(lagpm_ctx* ctx, void* dst, const void* src, size_t bytes, hipStream_t s);
 // Several such copies in one go (transfer.hip).
 struct lagpm_segment {

@@ -12,8 +12,8 @@
 // MI355X design (not the reference's): one global octree per box instead of one tree per
 // 4x4x4 cell. Particles are sorted by a 48-bit Morton key; the chaining cells are the
 // octree nodes of level L (2^L per axis, width n/2^L >= cutoff). A node is the run of
-// particles sharing a key prefix; nodes are numbered in pre-order by (first particle, level),
-// which a per-particle count + exclusive scan produces without any level-by-level pass.
+// particles sharing a key prefix. All levels are built at once: the keys around a particle say which
+// nodes begin at it, and the records stand level by level, the children of a node consecutive.
 // Target groups are subtrees of <= 128 particles; one wavefront walks the 27 neighbouring
 // cell trees for its group with a group-conservative opening test, stages accepted nodes
 // and opened leaves in LDS, and evaluates the interactions lane-per-target.
@@ -455,17 +455,12 @@ __global__ void __launch_bounds__(TB_THREADS) tree_emit_kernel(const uint64_t* _
         };
         uint32_t pre = wcnt[sq][nlev];
         for (int j = 0; j < nlev; j++) pre += below(__ballot(l1[q] <= L + j && L + j <= lk[q]));
-        unsigned long long m = __ballot(l1[q] <= L && L <= lk[q]);
-        uint32_t r = wcnt[sq][0] + below(m);
+        uint32_t r = wcnt[sq][0] + below(__ballot(l1[q] <= L && L <= lk[q]));
         for (int j = 0; j < nlev; j++) {
             const int l = L + j;
             const bool act = l1[q] <= l && l <= lk[q];
-            unsigned long long mn = 0ull;
             uint32_t rn = 0u;
-            if (j + 1 < nlev) {
-                mn = __ballot(l1[q] <= l + 1 && l + 1 <= lk[q]);
-                rn = wcnt[sq][j + 1] + below(mn);
-            }
+            if (j + 1 < nlev) rn = wcnt[sq][j + 1] + below(__ballot(l1[q] <= l + 1 && l + 1 <= lk[q]));
             if (act) {
                 uint32_t count = 0u;
                 const bool leaf = l == lk[q];
@@ -492,7 +487,6 @@ __global__ void __launch_bounds__(TB_THREADS) tree_emit_kernel(const uint64_t* _
                     cellroot[compact3(cell) + (size_t)mcell * (compact3(cell >> 1) + (size_t)mcell * compact3(cell >> 2))] = (int)r;
                 }
             }
-            m = mn;
             r = rn;
         }
     }
@@ -979,7 +973,7 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
                                                                 int nbox, const float2* __restrict__ tab0,
                                                                 const float4* __restrict__ tab12, int* __restrict__ stacks,
                                                                 unsigned* __restrict__ ticket_ctr) {
-    // positions are in scaled units (tree_prep_kernel): for the log tables r^2 here is lam r^2
+    // positions are in scaled units (tree_count_kernel): for the log tables r^2 here is lam r^2
     constexpr float lam = 1.0f;
     // One 1024-thread workgroup per CU: the 16 waves share one LDS copy of the particle force
     // table (32 KB) next to their private interaction lists.
@@ -990,8 +984,8 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
     // Staged particles need three words (their masses are 1) and a node's third record three (its
     // fourth is the mass, kept beside the centre). With the log tables the LDS pipe is the bound
     // (90 % busy at 256^3) and 12-byte entries take fewer of its cycles than 16-byte ones: walk
-    // 12.95 -> 12.55 ms at 256^3, its last vector spills gone with them. The reference law is bound by its arithmetic: 3.76 -> 3.90 ms with them, so it
-    // keeps the aligned ones.
+    // 12.95 -> 12.55 ms at 256^3. The reference law is bound by its arithmetic (3.76 -> 3.90 ms with
+    // 12 bytes) and keeps 16.
     using psrc = std::conditional_t<LOGT, float3, float4>;
     __shared__ psrc s_pp[WALK_WAVES][64];
     __shared__ float4 s_pc[WALK_WAVES][2][64];
@@ -1033,14 +1027,13 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
     // has finished its range takes tickets from the next ranges in turn (work stealing), and a
     // wave leaves after finding all eight ranges exhausted.
     // A wave's first group of its own range is its rank there (the waves of one workgroup far apart, so
-    // that few groups spread over all CUs), without an atomic, and later ones
-    // come from the range's counter, each counter in a cache line of its own. Once a range is found
-    // exhausted the workgroup's other waves skip it, and a range that the ranks alone cover is never
-    // asked for. Device-wide atomics on one line are served one after another: when every wave
-    // began with one and left by asking all eight ranges (of a 32^3 box's 741 groups: 33,000
-    // atomics for 4096 waves), their queue also held up the first loads of the waves that had a
-    // group, by 0.2 ms of its 0.63 ms walk, and 0.1 more went when 16 waves of a CU no
-    // longer began with neighbouring groups (first come had spread them). Walk times before and after: 32^3 0.63 -> 0.30 ms, 64^3
+    // that few groups spread over all CUs), without an atomic. Later ones come from the range's
+    // counter, each counter in a cache line of its own. Once a range is found exhausted the workgroup's
+    // other waves skip it, and a range that the ranks alone cover is never asked for. Device-wide
+    // atomics on one line are served one after another: when every wave began with one and left by
+    // asking all eight ranges (33,000 atomics for the 741 groups of a 32^3 box), their queue held up
+    // the first loads of the waves that had a group by 0.2 ms of a 0.63 ms walk. Spreading a
+    // workgroup's first groups took 0.1 more. Walk in ms before and after: 32^3 0.63 -> 0.30, 64^3
     // 0.75 -> 0.59, 100^3 1.47 -> 1.30, 128^3 2.14 -> 1.91, 256^3 13.94 -> 13.75.
     auto range_lo = [&](int x) -> int { return (int)(((long long)gtotal * x) / WALK_XCDS); };
     auto range_waves = [&](int x) -> int { return (((int)gridDim.x - x + WALK_XCDS - 1) / WALK_XCDS) * WALK_WAVES; };
@@ -1620,18 +1613,18 @@ __global__ void __launch_bounds__(WALK_THREADS) walk_f32_kernel(const walk_box* 
     }
 }
 
-// FP64 walk: the same tree, groups and criteria in FP64 throughout, one wavefront per target group.
-// It was one thread per target, depth first, each on its own path: 64 lanes then read 64 nodes and
-// 64 leaves of their own, from L2, and table lines too (theta = 0.5: 32^3 2.95 ms, 64^3 6.2, 128^3
-// 26.3; this: 0.50, 1.37, 5.0). Now a wave pops up to 64 nodes of its group's stack at a time, one per lane, and its targets share
-// the accepted nodes and the listed sources: sources are staged in LDS 64 at a time (those beyond the
-// cutoff from the group's box dropped), the pair term's table lines (value and slope, 80 KB) are in
-// LDS, and lane (slot, rep) sums every R-th source for its M targets. 16 waves and one table fill a
-// CU's LDS. A team of 1 or 4 waves takes a group: each wave walks down the same way until the
-// stack holds enough nodes, then keeps every S-th of them (before that it takes every S-th of the
-// accepted nodes and leaves), and the team's sums meet in LDS in a fixed order.
-// What bounds it: FP64 issue in the pair loop (about 20 operations a pair) for large
-// boxes, the heaviest group's own time for small ones.
+// FP64 walk: the same tree, groups and criteria in FP64 throughout, one wavefront per target group. (With
+// one thread per target, depth first, 64 lanes read 64 nodes and leaves of their own from L2, and table
+// lines too: theta = 0.5, 32^3 2.95 ms, 64^3 6.2, 128^3 26.3; this: 0.50, 1.37, 5.0.) A wave pops up to
+// 64 nodes of its group's stack at a time, one per lane, and its targets share the accepted nodes and
+// the listed sources. Sources are staged in LDS 64 at a time (those beyond the cutoff from the group's
+// box dropped), the pair term's table lines (value and slope, 80 KB) are in LDS, and lane (slot, rep)
+// sums every R-th source for its M targets. 16 waves and one table fill a CU's LDS. A team of 1 or 4
+// waves takes a group: each wave walks down the same way until the stack holds enough nodes, then
+// keeps every S-th of them (before that it takes every S-th of the accepted nodes and leaves), and the
+// team's sums meet in LDS in a fixed order.
+// What bounds it: FP64 issue in the pair loop (about 20 operations a pair) for large boxes, the
+// heaviest group's own time for small ones.
 struct walk64_args {
     const double *x, *y, *z;
     const int4* link;  // first particle, count, first child record, children
@@ -2201,7 +2194,7 @@ int lagpm_tree_walk_f32(lagpm_ctx* ctx, lagpm_box* const* boxes, const double* f
         A.cell_shift = 3 * (LAGPM_KEY_BITS - box->level_cell);
         A.mcell = box->mcell;
         A.naccept = LAGPM_NACCEPT;
-        // lengths in the units of pp (scaled by sc, see tree_prep_kernel)
+        // lengths in the units of pp (scaled by sc, see tree_count_kernel)
         const double sc = lagpm_tree_scale(box);
         A.box = (float)(box->p.n * sc);
         A.rc2 = (float)(box->p.rsphere * box->p.rsphere * sc * sc);
@@ -2391,7 +2384,7 @@ size_t lagpm_walk_stack_entries(int num_cu) {
 }
 
 // The octree of the last build in the box's own units: FP32 trees keep positions scaled by the
-// tree scale s (see tree_prep_kernel) and masses in particle masses; the FP64 tree keeps cells.
+// tree scale s (see tree_count_kernel) and masses in particle masses; the FP64 tree keeps cells.
 extern "C" int lagpm_tree_nodes_get(lagpm_ctx* ctx, lagpm_box* box, size_t cap, size_t* nnodes, int32_t* info,
                                     double* com, double* quad, uint32_t* order) {
     if (!ctx || !box || !nnodes) return lagpm_fail(ctx, LAGPM_E_INVAL, "NULL argument");
