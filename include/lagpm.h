@@ -334,9 +334,9 @@ int lagpm_kdk_step(lagpm_ctx* ctx, lagpm_box* box, double anow, double astep);
 int lagpm_batch_step(lagpm_ctx* ctx, lagpm_box* const* boxes, int nbox, const double* anow, const double* astep);
 /* Off: the steps that follow record their phase events (lagpm_box_timings); on, and without a call:
  * they do not. Every kernel of a step is launched either way, with the same results. (A call that
- * turned them on had steps replay captured hipGraphs. That was the slower path, and one process that
- * captured and replayed many ended in a segmentation fault on the host, of which no cause was found:
- * it has been taken out.) */
+ * turned them on had steps replay captured hipGraphs. That was the slower path, and two processes that
+ * captured and replayed many, one of them under a profiler, ended in a segmentation fault on the host,
+ * of which no cause was found: it has been taken out.) */
 int lagpm_set_step_graphs(lagpm_ctx* ctx, int enable);
 /* FP32 walks also count the evaluated particle pairs that are within the cutoff
  * (lagpm_tree_stats.n_pp_within): the useful fraction of the interaction lists. Costs a compare
